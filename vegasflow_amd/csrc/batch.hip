@@ -22,8 +22,9 @@ namespace mv {
 
 template <bool MIXED, int FAM, bool TRAIN>
 __device__ __forceinline__ void batch_events(const mv_batch_item& it, const mv_batch_tile& tile,
-                                             uint32_t draw, const void* tab, const void* tw,
-                                             const JacGroups& cs, double* hist, int nb, double* row) {
+                                             uint32_t draw, const void* tab,
+                                             const JacGroups<typename std::conditional<MIXED, float, double>::type>& cs,
+                                             double* hist, int nb, double* row) {
   using T = typename std::conditional<MIXED, float, double>::type;
   Integrand<T, FAM> F(it.fn);
   const Key key{(uint32_t)(it.seed & 0xffffffffu), (uint32_t)(it.seed >> 32)};
@@ -43,8 +44,7 @@ __device__ __forceinline__ void batch_events(const mv_batch_item& it, const mv_b
                                     static_cast<const float2*>(tab), cs, wh, nullptr, wscale);
     else
       tmp = event_f64<FAM, TRAIN>(F, lo0 + (uint32_t)k, hi, draw, key, groups, d,
-                                  static_cast<const double2*>(tab), static_cast<const double*>(tw), wh,
-                                  nullptr, wscale);
+                                  static_cast<const double2*>(tab), cs, wh, nullptr, wscale);
     acc += tmp;
     acc2 += tmp * tmp;
   }
@@ -60,20 +60,18 @@ __device__ __forceinline__ void batch_tile(const mv_batch_item& it, const mv_bat
   const int d = it.n_dim;
   const int nb = d * kBins;
   T2* tab = reinterpret_cast<T2*>(smem);
-  // the mixed table has no W column (fused_event.hpp)
-  T* tw = MIXED ? nullptr : reinterpret_cast<T*>(smem + 2 * nbmax);
-  double* hist = smem + (MIXED ? nbmax : 3 * nbmax);
+  double* hist = smem + (MIXED ? nbmax : 2 * nbmax);
   __syncthreads();  // the previous tile is done with the LDS
-  build_table<T, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab, tw);
+  build_table<T, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab);
   if (it.train)
     for (int i = threadIdx.x; i < kWaves * nb; i += kBlock) hist[i] = 0.0;
-  const JacGroups cs = MIXED ? jacobian_groups<FAM>(it.fn, d, nullptr) : JacGroups{};
+  const JacGroups<T> cs = jacobian_groups<T, FAM>(it.fn, d, nullptr);
   __syncthreads();
   double* row = rows + it.row_offset;
   if (it.train)
-    batch_events<MIXED, FAM, true>(it, tile, draw, tab, tw, cs, hist, nb, row);
+    batch_events<MIXED, FAM, true>(it, tile, draw, tab, cs, hist, nb, row);
   else
-    batch_events<MIXED, FAM, false>(it, tile, draw, tab, tw, cs, hist, nb, row);
+    batch_events<MIXED, FAM, false>(it, tile, draw, tab, cs, hist, nb, row);
 }
 
 // FAM >= 0: every tile belongs to an item of that family (smaller register
@@ -105,7 +103,7 @@ __global__ __launch_bounds__(kBlock) void batch_fused(const mv_batch_item* __res
 }
 
 // Tiles with pair histograms (fused_event.hpp), BS threads. LDS = the map
-// table (mixed: nbmax float2; FP64: nbmax (P, Q) pairs and nbmax W), then
+// table (mixed: nbmax float2; FP64: nbmax double2), then
 // pair_cells(max_dim) doubles. Training items add one LDS atomic per pair of
 // dimensions; frozen items run the plain event body of their precision.
 template <int FAM, int BS, bool MIXED, int D = 0>
@@ -114,7 +112,7 @@ __device__ __forceinline__ void batch_tile_pairs(const mv_batch_item& it, const 
                                                  double* __restrict__ rows, double* smem, int nbmax) {
   const int d = D ? D : it.n_dim;  // D > 0: compiled for that n_dim (straight-line event body)
   // 16-byte aligned: nbmax * 8 is a multiple of 400
-  double* H = smem + (MIXED ? nbmax : 3 * nbmax);
+  double* H = smem + (MIXED ? nbmax : 2 * nbmax);
   __syncthreads();  // the previous tile is done with the LDS
   const Key key{(uint32_t)(it.seed & 0xffffffffu), (uint32_t)(it.seed >> 32)};
   const double wscale = 1.0 / (double)it.n_events;  // xjac, monte_carlo.py:224-227
@@ -125,12 +123,12 @@ __device__ __forceinline__ void batch_tile_pairs(const mv_batch_item& it, const 
   double acc = 0.0, acc2 = 0.0;
   if constexpr (MIXED) {
     float2* tab = reinterpret_cast<float2*>(smem);
-    build_table<float, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab, nullptr);
+    build_table<float, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab);
     if (it.train) {
       const int half = pair_cells(d) / 2;
       for (int i = threadIdx.x; i < half; i += BS) reinterpret_cast<double2*>(H)[i] = make_double2(0.0, 0.0);
     }
-    const JacGroups cs = jacobian_groups<FAM>(it.fn, d, nullptr);
+    const JacGroups<float> cs = jacobian_groups<float, FAM>(it.fn, d, nullptr);
     __syncthreads();
     Integrand<float, FAM> F(it.fn);
     if (it.train) {
@@ -150,8 +148,8 @@ __device__ __forceinline__ void batch_tile_pairs(const mv_batch_item& it, const 
     }
   } else {
     double2* tab = reinterpret_cast<double2*>(smem);
-    double* tw = smem + 2 * nbmax;
-    build_table<double, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab, tw);
+    build_table<double, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab);
+    const JacGroups<double> cs = jacobian_groups<double, FAM>(it.fn, d, nullptr);
     if (it.train)
       for (int i = threadIdx.x; i < pair_cells(d); i += BS) H[i] = 0.0;
     __syncthreads();
@@ -159,14 +157,14 @@ __device__ __forceinline__ void batch_tile_pairs(const mv_batch_item& it, const 
     if (it.train) {
       for (int k = threadIdx.x; k < tile.count; k += BS) {
         const double tmp = event_f64<FAM, true, true, 0>(F, lo0 + (uint32_t)k, hi, draw, key, groups, d,
-                                                          tab, tw, H, nullptr, wscale);
+                                                          tab, cs, H, nullptr, wscale);
         acc += tmp;
         acc2 += tmp * tmp;
       }
     } else {
       for (int k = threadIdx.x; k < tile.count; k += BS) {
         const double tmp = event_f64<FAM, false, false, 0>(F, lo0 + (uint32_t)k, hi, draw, key, groups, d,
-                                                            tab, tw, nullptr, nullptr, wscale);
+                                                            tab, cs, nullptr, nullptr, wscale);
         acc += tmp;
         acc2 += tmp * tmp;
       }
@@ -275,7 +273,7 @@ extern "C" int mv_batch_fused(const mv_batch_item* items, int32_t n_items, const
   hipStream_t s = as_stream(stream);
   const bool mixed = precision == MV_MIXED;
   const size_t lds = mixed ? (size_t)(nbmax + kWaves * nbmax) * sizeof(double)
-                           : (size_t)(3 * nbmax + kWaves * nbmax) * sizeof(double);
+                           : (size_t)(2 * nbmax + kWaves * nbmax) * sizeof(double);
 #define MV_BF(MX, F)                                                                                \
   hipLaunchKernelGGL((batch_fused<MX, F>), dim3(blocks), dim3(kBlock), lds, s, items, tiles, n_tiles, \
                      nbmax, draws, grids, rows)
@@ -299,7 +297,7 @@ constexpr int kBatchPairBlock = 1024;
 
 size_t batch_pairs_lds(int max_dim, bool mixed) {
   if (max_dim < 1 || max_dim > kPairMaxDim) return 0;
-  const size_t table = (size_t)max_dim * kBins * (mixed ? 1 : 3);
+  const size_t table = (size_t)max_dim * kBins * (mixed ? 1 : 2);
   const size_t lds = (table + pair_cells(max_dim)) * sizeof(double);
   return lds <= max_lds_per_block() ? lds : 0;
 }

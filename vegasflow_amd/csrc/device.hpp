@@ -55,15 +55,31 @@ __device__ __forceinline__ uint32_t word(const uint4& v, int q) {
   return q == 0 ? v.x : (q == 1 ? v.y : (q == 2 ? v.z : v.w));
 }
 
+// The double in [1, 2) whose 52 mantissa bits are the top 52 bits of hi:lo.
+__device__ __forceinline__ double draw_mantissa(uint32_t hi, uint32_t lo) {
+  const uint32_t mlo = __builtin_amdgcn_alignbit(hi, lo, 12);      // (hi:lo) >> 12, low word
+  const uint32_t mhi = __builtin_amdgcn_alignbit(0x3FFu, hi, 12);  // 0x3FF00000 | (hi >> 12)
+  return __hiloint2double((int)mhi, (int)mlo);
+}
+
 // FP64 draw in [TECH_CUT, 1 - TECH_CUT]. The 52 mantissa bits of a double
 // in [1, 2) are the top 52 bits of the 64-bit word hi:lo, r = that - 1 in
 // [0, 1) (exact), then r * span + TECH_CUT as tf.random.uniform orders it
 // (monte_carlo.py:264-266).
 __device__ __forceinline__ double draw_f64(uint32_t hi, uint32_t lo) {
-  const uint32_t mlo = __builtin_amdgcn_alignbit(hi, lo, 12);  // (hi:lo) >> 12, low word
-  const uint32_t mhi = 0x3FF00000u | (hi >> 12);
-  const double r = __hiloint2double((int)mhi, (int)mlo) - 1.0;
-  return r * kSpan + kTechCut;
+  return (draw_mantissa(hi, lo) - 1.0) * kSpan + kTechCut;
+}
+
+// The position xn = 50 (1 - u) of the FP64 draw hi:lo in the unit interval of
+// 50 bins (vflow.py:117), for the fused kernels: 2 - m = 1 - r is exact, so
+// xn = fma(50 span, 1 - r, 50 (1 - TECH_CUT - span)) has one rounding where u,
+// 1 - u and the product with 50 have four: two FP64 operations for five, and
+// nearer to the real number (against 80-bit arithmetic rms 2.7e-15 and at most
+// 5.8e-15, the four roundings 2.9e-15 and 8.0e-15; the bins of the two forms
+// differ only where xn is within that of an edge). Always inside (0, 50).
+__device__ __forceinline__ double position_f64(uint32_t hi, uint32_t lo) {
+  constexpr double kEnd = kFBins * ((1.0 - kTechCut) - kSpan);  // xn of r = 1: 50 TECH_CUT
+  return fma(2.0 - draw_mantissa(hi, lo), kFBins * kSpan, kEnd);
 }
 
 // Mixed-precision position of a draw in one dimension, from the 32-bit word

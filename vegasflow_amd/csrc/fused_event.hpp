@@ -2,15 +2,15 @@
 // their LDS tables, shared by the single-integral and the batched kernels.
 //
 // Per (dimension, bin) the LDS table holds the map frac -> y = P + Q frac of
-// the integrand coordinate (Integrand::fold, integration limits folded in)
-// and, in FP64, the Jacobian factor W = dx * 50 (vflow.py:73, 78). The FP32
-// table of the mixed path is indexed by the mirrored bin k = 49 - bin and
-// takes 1 + mfrac, mfrac = 1 - frac (mixed_mirrored), so entry k holds
-// (P + 2Q, -Q): y = (P + 2Q) - Q (1 + mfrac) = P + Q frac. It has no W
-// column: W = Q * c_j with the per-dimension constant c_j = 50 / (xdelta_j *
-// fold scale_j) (jacobian_scale), so an event multiplies its slopes Q_j
-// and, after each group of four dimensions, the product of that group's c_j
-// (jacobian_groups), instead of one more LDS read per dimension.
+// the integrand coordinate (Integrand::fold, integration limits folded in).
+// The FP32 table of the mixed path is indexed by the mirrored bin k = 49 - bin
+// and takes 1 + mfrac, mfrac = 1 - frac (mixed_mirrored), so entry k holds
+// (P + 2Q, -Q): y = (P + 2Q) - Q (1 + mfrac) = P + Q frac. The Jacobian
+// factor W = dx * 50 (vflow.py:73, 78) has no column of its own: W = Q * c_j
+// with the per-dimension constant c_j = 50 / (xdelta_j * fold scale_j)
+// (jacobian_scale), so an event multiplies its slopes Q_j and, after each
+// group of dimensions, the product of that group's c_j (jacobian_groups),
+// instead of one more LDS read and address per dimension.
 #pragma once
 
 #include <type_traits>
@@ -24,8 +24,7 @@ __device__ __forceinline__ int clamp_bin(int b) { return b < 0 ? 0 : (b > kBins 
 template <typename T, int FAM>
 __device__ __forceinline__ void build_table(const mv_integrand& fn, const double* __restrict__ grid,
                                             int d, const double* xmin, const double* xdelta,
-                                            typename std::conditional<sizeof(T) == 8, double2, float2>::type* tab,
-                                            T* tw) {
+                                            typename std::conditional<sizeof(T) == 8, double2, float2>::type* tab) {
   const int nb = d * kBins;
   for (int i = threadIdx.x; i < nb; i += blockDim.x) {
     const int j = i / kBins, b = i - j * kBins;
@@ -44,39 +43,46 @@ __device__ __forceinline__ void build_table(const mv_integrand& fn, const double
       tab[i].x = (T)P;
       tab[i].y = (T)Q;
     }
-    if (tw) tw[i] = (T)(dx * kFBins);  // vflow.py:78
   }
 }
 
-// c_j of the mixed path's Jacobian: W = dx * 50 = Q * c_j. A dimension of
+// c_j of the Jacobian: W = dx * 50 = Q * c_j. A dimension of
 // zero width (xmin == xmax, allowed by monte_carlo.py:171) has Q = 0 and
 // takes c_j = 0, so its events weigh 0 as in FP64 (w * prod(xdelta) = 0).
 template <int FAM>
 __device__ __forceinline__ double jacobian_scale(const mv_integrand& fn, int j, const double* xdelta) {
-  const double xd = xdelta ? xdelta[j] : 1.0;
+  const double xd = xdelta[j];
   if (xd == 0.0) return 0.0;
-  return kFBins / (xd * Integrand<float, FAM>::fold_scale(fn, j));
+  return kFBins / (xd * Integrand<double, FAM>::fold_scale(fn, j));
 }
 
-// Products of c_j per group of four dimensions (g[k] for dimensions 4k ..
-// 4k + 3), each formed in FP64 and rounded once. An event multiplies its
+// Products of c_j per group of dimensions (g[k] for dimensions S k ..
+// S k + S - 1), each formed in FP64 and rounded once. An event multiplies its
 // slopes Q_j and, after each group, that group's product, so the running
-// FP32 product never strays from the Jacobian prod (dx_j * 50) of the
-// dimensions done by more than one group's factor. (One product of all the
-// c_j overflows FP32 with narrow limits: 500^16 on [0, 0.1]^16, against a
-// Jacobian of order 1.) Exact in range while every |log2 c_j| < 30.
+// product never strays from the Jacobian prod (dx_j * 50) of the dimensions
+// done by more than one group's factor. (One product of all the c_j overflows
+// FP32 with narrow limits: 500^16 on [0, 0.1]^16, against a Jacobian of order
+// 1.) FP32: groups of S = 4, in range while every |log2 c_j| < 30. FP64: pairs,
+// in range while every |log2 c_j| < 500, so wherever prod(xdelta) is.
+template <typename T>
 struct JacGroups {
-  float g[4];
+  static constexpr int S = sizeof(T) == 8 ? 2 : 4;
+  T g[MV_FUSED_MAX_DIM / S];
 };
 
-template <int FAM>
-__device__ __forceinline__ JacGroups jacobian_groups(const mv_integrand& fn, int d, const double* xdelta) {
-  JacGroups c;
+template <typename T, int FAM>
+__device__ __forceinline__ JacGroups<T> jacobian_groups(const mv_integrand& fn, int d, const double* xdelta) {
+  JacGroups<T> c;
+  constexpr int S = JacGroups<T>::S;
+  // without limits every c_j is the same (the fold scale is): one division
+  const double c0 = xdelta ? 0.0 : kFBins / Integrand<double, FAM>::fold_scale(fn, 0);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < MV_FUSED_MAX_DIM / S; ++k) {
     double p = 1.0;
-    for (int j = 4 * k; j < 4 * k + 4 && j < d; ++j) p *= jacobian_scale<FAM>(fn, j, xdelta);
-    c.g[k] = (float)p;
+#pragma unroll
+    for (int j = S * k; j < S * k + S; ++j)
+      if (j < d) p *= xdelta ? jacobian_scale<FAM>(fn, j, xdelta) : c0;
+    c.g[k] = (T)p;
   }
   return c;
 }
@@ -130,28 +136,35 @@ __device__ __forceinline__ double pair_marginal_half(const double* H, int m, int
   return a;
 }
 
-template <bool PAIRS>
-__device__ __forceinline__ void event_hist(double* wh, const uint32_t (&pk)[4], int d, double tmp2) {
-  if (PAIRS)
-    pair_adds(wh, pk, d, tmp2);
-  else
-    hist_adds(wh, pk, d, tmp2);
+// The same from the byte offset of the event's cell within each pair table
+// (one multiply-add per pair of dimensions, no packed bins to take apart).
+template <int N>
+__device__ __forceinline__ void pair_cell_adds(double* H, const uint32_t (&cell)[N], int d, double tmp2) {
+  char* Hb = reinterpret_cast<char*>(H);
+#pragma unroll
+  for (int p = 0; p < kPairMaxDim / 2; ++p)
+    if (2 * p < d) lds_add(reinterpret_cast<double*>(Hb + p * kPairBins * sizeof(double) + cell[p]), tmp2);
 }
 
 // One event, FP64 (vflow.py:87-126 + 33-83 + 389-430). Returns tmp = w f
 // and, when training, adds tmp^2 to the histogram ``wh`` (the wave's
 // per-dimension histograms, or the workgroup's pair histograms if PAIRS).
+// Philox draws take position_f64, injected ones the reference's operation
+// order (they may be any uniform, also outside TECH_CUT: the bin is clamped).
 // INJ: injected draws taken when inj != nullptr (-1, tested per event), never
 // (0) or always (1); a compile-time 0 or 1 leaves no test in the event body.
 template <int FAM, bool TRAIN, bool PAIRS = false, int INJ = -1>
 __device__ __forceinline__ double event_f64(Integrand<double, FAM>& F, uint32_t c0, uint32_t c1,
                                             uint32_t draw, Key key, int groups, int d,
-                                            const double2* tab, const double* tw, double* wh,
+                                            const double2* tab, const JacGroups<double>& cs, double* wh,
                                             const double* inj, double wscale) {
   const bool injected = INJ < 0 ? inj != nullptr : INJ > 0;
   F.begin();
   double w = 1.0;
   uint32_t pk[4] = {0u, 0u, 0u, 0u};
+  uint32_t cell[kPairMaxDim / 2 + 1];  // byte offsets of the event's pair cells
+#pragma unroll
+  for (int p = 0; p <= kPairMaxDim / 2; ++p) cell[p] = 0u;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     if (g < groups) {
@@ -164,29 +177,32 @@ __device__ __forceinline__ double event_f64(Integrand<double, FAM>& F, uint32_t 
       for (int q = 0; q < 4; ++q) {
         const int j = 4 * g + q;
         if (j < d) {
-          const double u = injected ? inj[j] : draw_f64(word(h, q), word(l, q));
-          const double xn = kFBins * (1.0 - u);  // vflow.py:117
-          const int ind = clamp_bin((int)xn);    // vflow.py:67
+          const double xn = injected ? kFBins * (1.0 - inj[j]) : position_f64(word(h, q), word(l, q));  // vflow.py:117
+          const int ind = injected ? clamp_bin((int)xn) : (int)xn;  // vflow.py:67
           const double2 t = tab[j * kBins + ind];
-          const double frac = xn - floor(xn);    // vflow.py:75
+          const double frac = injected ? xn - floor(xn) : __builtin_amdgcn_fract(xn);  // vflow.py:75
           F.add_folded(j, fma(t.y, frac, t.x));  // vflow.py:76
-          w = w * tw[j * kBins + ind];           // vflow.py:78
-          if (TRAIN) pk[g] |= (uint32_t)ind << (8 * q);
+          w = w * t.y;                           // vflow.py:78, with cs
+          if (q & 1) w = w * cs.g[2 * g + (q >> 1)];
+          if (TRAIN && PAIRS) cell[2 * g + (q >> 1)] += (uint32_t)ind * (q & 1 ? 8u : 8u * kBins);
+          if (TRAIN && !PAIRS) pk[g] |= (uint32_t)ind << (8 * q);
         }
       }
     }
   }
+  if (d & 1) w = w * cs.g[d >> 1];
   const double tmp = (w * wscale) * F.value();  // vflow.py:416
-  if (TRAIN) event_hist<PAIRS>(wh, pk, d, tmp * tmp);  // vflow.py:417, 370-387
+  if (TRAIN && PAIRS) pair_cell_adds(wh, cell, d, tmp * tmp);  // vflow.py:417, 370-387
+  if (TRAIN && !PAIRS) hist_adds(wh, pk, d, tmp * tmp);
   return tmp;
 }
 
 // One event, mixed precision: FP32 map and integrand from the high word of
 // each draw (mixed_mirrored), FP64 result.
-template <int FAM, bool TRAIN, bool PAIRS = false, int INJ = -1>
+template <int FAM, bool TRAIN, int INJ = -1>
 __device__ __forceinline__ double event_mixed(Integrand<float, FAM>& F, uint32_t c0, uint32_t c1,
                                               uint32_t draw, Key key, int groups, int d,
-                                              const float2* tab, const JacGroups& cs, double* wh,
+                                              const float2* tab, const JacGroups<float>& cs, double* wh,
                                               const uint32_t* inj, double wscale) {
   const bool injected = INJ < 0 ? inj != nullptr : INJ > 0;
   F.begin();
@@ -215,7 +231,7 @@ __device__ __forceinline__ double event_mixed(Integrand<float, FAM>& F, uint32_t
   // w * f in FP32; the 1/N (and limits) factor in FP64 so that its rounding
   // is not a systematic bias
   const double tmp = (double)(w * F.value()) * wscale;
-  if (TRAIN) event_hist<PAIRS>(wh, pk, d, tmp * tmp);
+  if (TRAIN) hist_adds(wh, pk, d, tmp * tmp);
   return tmp;
 }
 
@@ -256,7 +272,7 @@ __device__ __forceinline__ void pair_dim(Integrand<float, FAM>& F, int j, uint32
 template <int FAM, bool INJ>
 __device__ __forceinline__ double event_mixed_pairs(Integrand<float, FAM>& F, uint32_t c0, uint32_t c1,
                                                     uint32_t draw, Key key, int d, const float2* tab,
-                                                    const JacGroups& cs, double* H, const uint32_t* inj,
+                                                    const JacGroups<float>& cs, double* H, const uint32_t* inj,
                                                     double wscale) {
   F.begin();
   float w = 1.0f;
@@ -289,11 +305,7 @@ __device__ __forceinline__ double event_mixed_pairs(Integrand<float, FAM>& F, ui
     }
   }
   const double tmp = (double)(w * F.value()) * wscale;
-  const double tmp2 = tmp * tmp;
-  char* Hb = reinterpret_cast<char*>(H);
-#pragma unroll
-  for (int p = 0; p < kPairMaxDim / 2; ++p)
-    if (2 * p < d) lds_add(reinterpret_cast<double*>(Hb + p * kPairBins * sizeof(double) + cell[p]), tmp2);
+  pair_cell_adds(H, cell, d, tmp * tmp);
   return tmp;
 }
 

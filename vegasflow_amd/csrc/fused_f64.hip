@@ -3,11 +3,10 @@
 // (integrand family, train, n_dim) so that the event body is straight-line
 // code for the n_dim of the launch.
 //
-// Per event: Philox draws (two words per dimension), bin and fraction in the
-// reference's FP64 operation order, the folded (P, Q, W) table in LDS, the
-// integrand, w f sums; when training, (w f)^2 into the wave's private LDS
-// histogram (kWaves copies of n_dim x 50 doubles). LDS: 3 + 4 (training)
-// doubles per (dimension, bin).
+// Per event: Philox draws (two words per dimension), position_f64, the folded
+// (P, Q) table in LDS, the integrand, w f sums; when training, (w f)^2 into
+// the wave's private LDS histogram (kWaves copies of n_dim x 50 doubles).
+// LDS (static): 2 + 4 (training) doubles per (dimension, bin).
 #include <array>
 #include <utility>
 
@@ -22,12 +21,12 @@ template <int FAM, bool TRAIN, int D, bool INJ>
 __global__ __launch_bounds__(kBlock) void vegas_fused_f64(StepK s, mv_integrand fn,
                                                           const double* __restrict__ grid, RowsK R) {
   const uint32_t draw = draw_of(s);
-  extern __shared__ double smem[];
   constexpr int nb = D * kBins;
+  __shared__ __align__(16) double smem[(2 + (TRAIN ? kWaves : 0)) * nb];
   double2* tab = reinterpret_cast<double2*>(smem);
-  double* tw = smem + 2 * nb;
-  double* hist = tw + nb;
-  build_table<double, FAM>(fn, grid, D, s.xmin, s.xdelta, tab, tw);
+  double* hist = smem + 2 * nb;
+  build_table<double, FAM>(fn, grid, D, s.xmin, s.xdelta, tab);
+  const JacGroups<double> cs = jacobian_groups<double, FAM>(fn, D, s.xdelta);
   if (TRAIN)
     for (int i = threadIdx.x; i < kWaves * nb; i += kBlock) hist[i] = 0.0;
   __syncthreads();
@@ -36,13 +35,21 @@ __global__ __launch_bounds__(kBlock) void vegas_fused_f64(StepK s, mv_integrand 
   const double* inj = static_cast<const double*>(s.inject);
   const double wscale = s.xmin ? s.xjac * s.xdeltajac : s.xjac;  // monte_carlo.py:270-274
   double acc = 0.0, acc2 = 0.0;
-  const int64_t step = (int64_t)gridDim.x * kBlock;
-  for (int64_t i = spread_first_event(); i < s.n_events; i += step) {
-    const double tmp = event_f64<FAM, TRAIN, false, INJ ? 1 : 0>(
-        F, s.ev_lo + (uint32_t)i, s.ev_hi, draw, s.key, (D + 3) / 4, D, tab, tw, wh,
-        INJ ? inj + i * D : nullptr, wscale);
-    acc += tmp;
-    acc2 += tmp * tmp;
+  if (INJ) {
+    const int64_t step = (int64_t)gridDim.x * kBlock;
+    for (int64_t i = spread_first_event(); i < s.n_events; i += step) {
+      const double tmp = event_f64<FAM, TRAIN, false, 1>(F, 0u, 0u, 0u, s.key, (D + 3) / 4, D, tab, cs, wh,
+                                                         inj + i * D, wscale);
+      acc += tmp;
+      acc2 += tmp * tmp;
+    }
+  } else {
+    event_trips<kBlock>(s, [&](uint32_t c) {
+      const double tmp = event_f64<FAM, TRAIN, false, 0>(F, c, s.ev_hi, draw, s.key, (D + 3) / 4, D, tab, cs, wh,
+                                                         nullptr, wscale);
+      acc += tmp;
+      acc2 += tmp * tmp;
+    });
   }
   finish_block<TRAIN>(acc, acc2, hist, nb, R);
 }
@@ -67,10 +74,8 @@ int launch_fam(const StepK& k, const mv_integrand& fn, const double* grid, const
   if (k.n_dim < 1 || k.n_dim > MV_FUSED_MAX_DIM)
     return fail(MV_ERR_UNSUPPORTED, "fused FP64 kernel: n_dim %d outside 1..%d", k.n_dim,
                 MV_FUSED_MAX_DIM);
-  const int nb = k.n_dim * kBins;
-  const size_t lds = (size_t)(3 * nb + (TRAIN ? kWaves * nb : 0)) * sizeof(double);
   const Kernel kern = (k.inject ? table_inj : table)[k.n_dim - 1];
-  return launch_producer(kern, k.n_events, lds, st, k, fn, grid, R);
+  return launch_producer(kern, k.n_events, 0, st, k, fn, grid, R);
 }
 
 }  // namespace

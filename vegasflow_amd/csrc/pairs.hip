@@ -28,47 +28,31 @@ __global__ __launch_bounds__(kPairBlock) void vegas_fused_pairs(StepK s, mv_inte
   __shared__ __align__(16) double smem[nb + pair_cells(D)];
   float2* tab = reinterpret_cast<float2*>(smem);
   double* H = smem + nb;  // 16-byte aligned: nb * 8 is a multiple of 400
-  build_table<float, FAM>(fn, grid, D, s.xmin, s.xdelta, tab, nullptr);
+  build_table<float, FAM>(fn, grid, D, s.xmin, s.xdelta, tab);
   constexpr int half = pair_cells(D) / 2;
   for (int i = threadIdx.x; i < half; i += kPairBlock)
     reinterpret_cast<double2*>(H)[i] = make_double2(0.0, 0.0);
-  const JacGroups cs = jacobian_groups<FAM>(fn, D, s.xdelta);
+  const JacGroups<float> cs = jacobian_groups<float, FAM>(fn, D, s.xdelta);
   __syncthreads();
   Integrand<float, FAM> F(fn);
   const uint32_t* inj = static_cast<const uint32_t*>(s.inject);
   const double wscale = s.xmin ? s.xjac * s.xdeltajac : s.xjac;  // monte_carlo.py:270-274
   double acc = 0.0, acc2 = 0.0;
-  const int64_t step = (int64_t)gridDim.x * kPairBlock;
-  const int64_t i0 = spread_first_event();
   if (inj) {
-    for (int64_t i = i0; i < s.n_events; i += step) {
+    const int64_t step = (int64_t)gridDim.x * kPairBlock;
+    for (int64_t i = spread_first_event(); i < s.n_events; i += step) {
       const double tmp = event_mixed_pairs<FAM, true>(F, 0u, 0u, 0u, s.key, D, tab, cs, H,
                                                       inj + i * D, wscale);
       acc += tmp;
       acc2 += tmp * tmp;
     }
   } else {
-    // The wave's trips in which all 64 lanes have an event run without a
-    // per-lane test, counted on the scalar unit; at most one trip with a
-    // per-lane test follows. The Philox counter word advances by the step
-    // (mod 2^32) as the 64-bit event index would.
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int64_t w0 = ((int64_t)wave * gridDim.x + blockIdx.x) * 64;  // the wave's first event (i0 - lane)
-    const int64_t full = s.n_events - 64 - w0 >= 0 ? (s.n_events - 64 - w0) / step + 1 : 0;
-    uint32_t c = s.ev_lo + (uint32_t)i0;
-    for (int64_t t = 0; t < full; ++t) {
+    event_trips<kPairBlock>(s, [&](uint32_t c) {
       const double tmp = event_mixed_pairs<FAM, false>(F, c, s.ev_hi, draw, s.key, D, tab, cs, H, nullptr,
                                                        wscale);
       acc += tmp;
       acc2 += tmp * tmp;
-      c += (uint32_t)step;
-    }
-    if (i0 + full * step < s.n_events) {
-      const double tmp = event_mixed_pairs<FAM, false>(F, c, s.ev_hi, draw, s.key, D, tab, cs, H, nullptr,
-                                                       wscale);
-      acc += tmp;
-      acc2 += tmp * tmp;
-    }
+    });
   }
   finish_pairs<kPairBlock, true, true>(acc, acc2, H, D, group_row(R));
 }

@@ -151,6 +151,27 @@ __device__ __forceinline__ int64_t spread_first_event() {
   return ((int64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x) * 64 + (threadIdx.x & 63);
 }
 
+// Runs ``body(counter word)`` for every event of this thread (the events of
+// spread_first_event, BS-thread workgroups). The wave's trips in which all 64
+// lanes have an event are counted on the scalar unit and run without a
+// per-lane test; at most one trip with a per-lane test follows. The Philox
+// counter word advances by the step (mod 2^32) as the 64-bit event index
+// would.
+template <int BS, typename Body>
+__device__ __forceinline__ void event_trips(const StepK& s, Body&& body) {
+  const int64_t step = (int64_t)gridDim.x * BS;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t w0 = ((int64_t)wave * gridDim.x + blockIdx.x) * 64;  // the wave's first event
+  const int64_t i0 = w0 + (threadIdx.x & 63);
+  const int64_t full = s.n_events - 64 - w0 >= 0 ? (s.n_events - 64 - w0) / step + 1 : 0;
+  uint32_t c = s.ev_lo + (uint32_t)i0;
+  for (int64_t t = 0; t < full; ++t) {
+    body(c);
+    c += (uint32_t)step;
+  }
+  if (i0 + full * step < s.n_events) body(c);
+}
+
 // this workgroup's group row
 __device__ __forceinline__ double* group_row(const RowsK& R) {
   return R.rows + (int64_t)(blockIdx.x % kRows) * R.stride;
@@ -247,10 +268,9 @@ int launch_vegas_fused_pairs(int family, const StepK& k, const mv_integrand& fn,
                              const RowsK& R, hipStream_t st);
 
 // The FP64 training producer with pair histograms (pairs_f64.hip), as
-// launch_vegas_fused_pairs; ``lds`` = fused_pairs_f64_lds(n_dim).
-size_t fused_pairs_f64_lds(int d);
+// launch_vegas_fused_pairs, with n_dim * 50 double2 table entries.
 int launch_vegas_fused_pairs_f64(int family, const StepK& k, const mv_integrand& fn, const double* grid,
-                                 const RowsK& R, size_t lds, hipStream_t st);
+                                 const RowsK& R, hipStream_t st);
 
 template <bool TRAIN, bool SUMS = true>
 __device__ __forceinline__ void finish_block(double acc, double acc2, const double* hist,

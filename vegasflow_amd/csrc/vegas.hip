@@ -525,22 +525,19 @@ extern "C" int32_t mv_producer_rows(int64_t n_events) {
 
 namespace {
 
-// LDS bytes of vegas_fused_pairs' table and cells (static in the kernel),
-// 0 where it does not apply (FP64, no training, n_dim outside
-// kPairMinDim..kPairMaxDim, or more LDS than a workgroup may have)
-size_t pairs_lds(int d, bool mixed, bool train) {
-  if (!mixed || !train || d < kPairMinDim || d > kPairMaxDim) return 0;
-  const size_t lds = (size_t)(d * kBins + pair_cells(d)) * sizeof(double);
-  return lds <= max_lds_per_block() ? lds : 0;
+// Whether a training step runs through pair tables: their LDS (static in the
+// kernels: the map table, then the cells) must be what a workgroup may have.
+bool pairs_apply(int d, bool mixed) {
+  return d >= kPairMinDim && d <= kPairMaxDim &&
+         (size_t)((mixed ? 1 : 2) * d * kBins + pair_cells(d)) * sizeof(double) <= max_lds_per_block();
 }
 
 template <int FAM>
 int launch_vegas_fused(const StepK& k, const mv_integrand& fn, bool mixed, bool train,
                        const double* grid, const RowsK& R, hipStream_t st) {
-  if (pairs_lds(k.n_dim, mixed, train) != 0) return launch_vegas_fused_pairs(FAM, k, fn, grid, R, st);
-  if (!mixed && train && k.n_dim >= kPairMinDim && k.n_dim <= kPairMaxDim &&
-      fused_pairs_f64_lds(k.n_dim) <= max_lds_per_block())
-    return launch_vegas_fused_pairs_f64(FAM, k, fn, grid, R, fused_pairs_f64_lds(k.n_dim), st);
+  if (train && pairs_apply(k.n_dim, mixed))
+    return mixed ? launch_vegas_fused_pairs(FAM, k, fn, grid, R, st)
+                 : launch_vegas_fused_pairs_f64(FAM, k, fn, grid, R, st);
   return mixed ? launch_vegas_fused_mixed(FAM, train, k, fn, grid, R, st)
                : launch_vegas_fused_f64(FAM, train, k, fn, grid, R, st);
 }
