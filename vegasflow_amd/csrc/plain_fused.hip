@@ -14,6 +14,57 @@
 
 namespace mv {
 
+// One draw per dimension as FP64 integrand coordinate y_j = P_j + Q_j r, r the
+// draw's 52 bits in [0, 1) (exact), for a compile-time n_dim: u = TECH_CUT +
+// span r, the integration limits (LIM, monte_carlo.py:271-274) and the
+// integrand's own affine map (Integrand::fold) in one FMA, where the separate
+// steps take up to seven operations (d = 8 Gaussian: 248 -> 207 VALU
+// instructions per 64 events, 75.2 -> 65.5 us at 1e7 events). P_j is held in scalar registers; without
+// limits Q_j is the same for every dimension.
+template <int FAM, int D, bool LIM>
+struct PlainMap {
+  double P[D], Q[LIM ? D : 1];
+  __device__ __forceinline__ PlainMap(const StepK& s, const mv_integrand& fn) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      double p = kTechCut, q = kSpan;
+      if (LIM) {
+        p = s.xmin[j] + kTechCut * s.xdelta[j];
+        q = kSpan * s.xdelta[j];
+      }
+      Integrand<double, FAM>::fold(fn, j, p, q);
+      P[j] = bcast_lane(p, 0);
+      if (LIM || j == 0) Q[LIM ? j : 0] = q;
+    }
+  }
+  __device__ __forceinline__ double operator()(int j, uint32_t hi, uint32_t lo) const {
+    return fma(draw_mantissa(hi, lo) - 1.0, Q[LIM ? j : 0], P[j]);
+  }
+};
+
+// The FP64 events of this thread for a compile-time n_dim and Philox draws.
+template <int FAM, int D, bool LIM>
+__device__ __forceinline__ void plain_events_f64(const StepK& s, const mv_integrand& fn, uint32_t draw,
+                                                 Integrand<double, FAM>& F, double wt, double& acc,
+                                                 double& acc2) {
+  const PlainMap<FAM, D, LIM> map(s, fn);
+  constexpr int groups = (D + 3) / 4;
+  event_trips<kBlock>(s, [&](uint32_t c0) {
+    F.begin();
+#pragma unroll
+    for (int g = 0; g < groups; ++g) {
+      const uint4 h = philox(c0, s.ev_hi, draw, (uint32_t)g, s.key);
+      const uint4 l = philox(c0, s.ev_hi, draw, (uint32_t)(groups + g), s.key);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (4 * g + q < D) F.add_folded(4 * g + q, map(4 * g + q, word(h, q), word(l, q)));
+    }
+    const double tmp = F.value() * wt;  // plain.py:27
+    acc += tmp;
+    acc2 += tmp * tmp;
+  });
+}
+
 // The events of this thread (plain.py:18-35): uniform points, with the
 // integration limits (LIM, monte_carlo.py:271-274) or without, the
 // integrand, and the sums of w f and (w f)^2. INJ: injected draws
@@ -24,9 +75,8 @@ __device__ __forceinline__ void plain_events(const StepK& s, uint32_t draw, Inte
                                              double& acc, double& acc2) {
   const int d = D ? D : s.n_dim;
   const int groups = D ? (D + 3) / 4 : s.groups;
-  const int64_t step = (int64_t)gridDim.x * kBlock;
-  for (int64_t i = spread_first_event(); i < s.n_events; i += step) {
-    const uint32_t c0 = s.ev_lo + (uint32_t)i, c1 = s.ev_hi;  // launch-uniform high word
+  const uint32_t c1 = s.ev_hi;  // launch-uniform high word
+  const auto event = [&](uint32_t c0, [[maybe_unused]] int64_t i) {
     F.begin();
 #pragma unroll
     for (int g = 0; g < groups; ++g) {
@@ -57,6 +107,12 @@ __device__ __forceinline__ void plain_events(const StepK& s, uint32_t draw, Inte
     const double tmp = (double)F.value() * wt;  // plain.py:27
     acc += tmp;
     acc2 += tmp * tmp;
+  };
+  if (INJ) {
+    const int64_t step = (int64_t)gridDim.x * kBlock;
+    for (int64_t i = spread_first_event(); i < s.n_events; i += step) event(0u, i);
+  } else {
+    event_trips<kBlock>(s, [&](uint32_t c0) { event(c0, 0); });
   }
 }
 
@@ -68,10 +124,16 @@ __global__ __launch_bounds__(kBlock) void plain_fused(StepK s, mv_integrand fn, 
   const bool limits = s.xmin != nullptr;
   const double wt = limits ? s.xjac * s.xdeltajac : s.xjac;  // monte_carlo.py:270-274
   double acc = 0.0, acc2 = 0.0;
-  if (limits)
+  if constexpr (!MIXED && !INJ && D > 0) {
+    if (limits)
+      plain_events_f64<FAM, D, true>(s, fn, draw, F, wt, acc, acc2);
+    else
+      plain_events_f64<FAM, D, false>(s, fn, draw, F, wt, acc, acc2);
+  } else if (limits) {
     plain_events<FAM, MIXED, D, INJ, true>(s, draw, F, wt, acc, acc2);
-  else
+  } else {
     plain_events<FAM, MIXED, D, INJ, false>(s, draw, F, wt, acc, acc2);
+  }
   finish_block<false>(acc, acc2, nullptr, 0, R);
 }
 
