@@ -74,7 +74,9 @@ def build(verbose=False, jobs=None):
             print(r.stderr, file=sys.stderr)
         return obj
 
-    jobs = jobs or min(len(srcs), max(1, (os.cpu_count() or 2) // 2), 8)
+    jobs = jobs or min(len(srcs), max(1, os.cpu_count() or 2), 8)
+    # the longest compiles (the VEGAS+ producers) first
+    srcs.sort(key=lambda f: "vplus_" not in os.path.basename(f))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
         objs = list(ex.map(compile_one, srcs))
     out = lib_path()

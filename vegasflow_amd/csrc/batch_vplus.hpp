@@ -1,10 +1,10 @@
-// batch_vplus.hip - the producer of batched VegasFlowPlus integrals
+// batch_vplus.hpp - the producer of batched VegasFlowPlus integrals
 // (mv_batch_vplus_fused): many VEGAS+ integrals advance one iteration in one
 // persistent launch (vflowplus.py:37-80 + 187-220 per item). The iteration
 // end of the items is in vplus.hip (mv_batch_vplus_finalize).
 //
 // Workgroups stride over tiles of consecutive events of one item. Per tile:
-// the item's map table (P, Q, W = dx * 50) in LDS, histograms zeroed, then
+// the item's map table in LDS, histograms zeroed, then
 // the tile's 64-event trips split evenly over the waves, each wave walking
 // its run with the single-integral event body (vplus_run: hypercube lookup
 // over the item's offsets, draws, map, integrand, per-cube segmented sums
@@ -13,6 +13,8 @@
 // upper bound of the adaptive event count) does nothing. Launches whose
 // items share n_dim run a kernel compiled for it (the registers of one event
 // body); mixed dimensions choose the body per tile.
+#pragma once
+
 #include <algorithm>
 #include <array>
 #include <type_traits>
@@ -32,32 +34,29 @@ namespace mv {
 // 2 <= D <= 14).
 template <bool MIXED, int FAM, bool TRAIN, bool PAIRS, int D>
 __device__ void vplus_tile_body(const mv_batch_vplus_item& it, const StepK& s, uint32_t draw,
-                                const StrataK& st, int64_t first, int64_t end, const void* tab_,
-                                const void* tw_, double* hist, double* __restrict__ ress,
-                                double* __restrict__ ress2, double& acc, double& acc2) {
+                                const StrataK& st, int64_t first, int64_t end, int c0,
+                                const VplusEntry<MIXED>* tab, double* hist, double* __restrict__ ress,
+                                double* __restrict__ ress2) {
   using T = typename std::conditional<MIXED, float, double>::type;
-  using T2 = typename std::conditional<MIXED, float2, double2>::type;
   constexpr bool P = PAIRS && D >= kPairMinDim && D <= kPairMaxDim;
   if (PAIRS && !P) return;  // a pair launch holds only items it can pair
   Integrand<T, FAM> F(it.fn);
-  const double fstrat = (double)st.n_strat;
-  const float rn = 1.0f / (float)st.n_strat;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   double* wh = P ? hist : hist + wave * (D * kBins);
-  vplus_run<FAM, TRAIN, MIXED, D, false, P>(F, s, draw, st, first, end, fstrat, 1.0 / fstrat, rn,
-                                            static_cast<const T2*>(tab_), static_cast<const T*>(tw_), s.xjac,
-                                            wh, ress, ress2, acc, acc2);
+  const JacGroups<double> cs = MIXED ? JacGroups<double>{} : jacobian_groups<double, FAM>(it.fn, D, nullptr);
+  const StrataPos<MIXED, false> sp(st.n_strat);
+  vplus_run<FAM, TRAIN, MIXED, D, false, P>(F, s, draw, st, sp, first, end, c0, tab, cs, s.xjac, wh, ress, ress2);
 }
 
 template <bool MIXED, int FAM, bool TRAIN, bool PAIRS, int... Ds>
 __device__ void vplus_tile_dispatch(std::integer_sequence<int, Ds...>, int d, const mv_batch_vplus_item& it,
                                     const StepK& s, uint32_t draw, const StrataK& st, int64_t first,
-                                    int64_t end, const void* tab, const void* tw, double* hist,
-                                    double* ress, double* ress2, double& acc, double& acc2) {
+                                    int64_t end, int c0, const VplusEntry<MIXED>* tab, double* hist,
+                                    double* ress, double* ress2) {
   // one call for the tile's n_dim (d is workgroup-uniform)
-  ((d == Ds + 1 ? vplus_tile_body<MIXED, FAM, TRAIN, PAIRS, Ds + 1>(it, s, draw, st, first, end, tab, tw, hist,
-                                                                    ress, ress2, acc, acc2)
-                : void()),
+  ((d == Ds + 1
+        ? vplus_tile_body<MIXED, FAM, TRAIN, PAIRS, Ds + 1>(it, s, draw, st, first, end, c0, tab, hist, ress, ress2)
+        : void()),
    ...);
 }
 
@@ -77,15 +76,12 @@ __global__ __launch_bounds__(BS) void batch_vplus_fused(const mv_batch_vplus_ite
                                                         double* __restrict__ ress,
                                                         double* __restrict__ ress2,
                                                         double* __restrict__ rows, int nbmax) {
-  using T = typename std::conditional<MIXED, float, double>::type;
-  using T2 = typename std::conditional<MIXED, float2, double2>::type;
   constexpr int W = BS / 64;
   extern __shared__ double smem[];
-  // LDS: table (nbmax T2), W column (nbmax T), histograms (per-wave, or the
-  // pair tables)
-  T2* tab = reinterpret_cast<T2*>(smem);
-  T* tw = reinterpret_cast<T*>(smem + (MIXED ? nbmax : 2 * nbmax));
-  double* hist = smem + (MIXED ? nbmax + (nbmax + 1) / 2 : 3 * nbmax);
+  // LDS: the map table (nbmax 16-byte entries), then the histograms (per-wave,
+  // or the pair tables)
+  VplusEntry<MIXED>* tab = reinterpret_cast<VplusEntry<MIXED>*>(smem);
+  double* hist = smem + 2 * nbmax;
   for (int t = blockIdx.x; t < n_tiles; t += gridDim.x) {
     const mv_batch_tile tile = tiles[t];
     const mv_batch_vplus_item& it = items[tile.item];
@@ -96,20 +92,14 @@ __global__ __launch_bounds__(BS) void batch_vplus_fused(const mv_batch_vplus_ite
     if (first >= end) continue;  // workgroup-uniform: no barrier skipped by part of it
     const int d = it.n_dim;
     const int nb = d * kBins;
+    // this wave's run: the tile's trips split evenly over the waves
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t trips = (end - first + 63) >> 6;
+    const int64_t a = first + trip_of(wave, trips, W) * 64;
+    const int64_t b = min(first + trip_of(wave + 1, trips, W) * 64, end);
+    const int c0 = a < b ? find_cube_wave(st.off, st.n_cubes, (int)a) : 0;
     __syncthreads();  // the previous tile is done with the LDS
-    const double* grid = grids + it.grid_offset;
-    for (int i = threadIdx.x; i < nb; i += BS) {
-      const int j = i / kBins, b = i - j * kBins;
-      const double lo = grid[j * (kBins + 1) + b];
-      const double dx = grid[j * (kBins + 1) + b + 1] - lo;  // vflow.py:73
-      double P = lo, Q = dx;
-      Integrand<T, FAM>::fold(it.fn, j, P, Q);
-      T2 e;
-      e.x = (T)P;
-      e.y = (T)Q;
-      tab[i] = e;
-      tw[i] = (T)(dx * kFBins);  // vflow.py:78
-    }
+    vplus_table<MIXED, FAM, BS>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab);
     const int hist_len = PAIRS ? pair_cells(d) : W * nb;
     if (it.train)
       for (int i = threadIdx.x; i < hist_len; i += BS) hist[i] = 0.0;
@@ -123,35 +113,27 @@ __global__ __launch_bounds__(BS) void batch_vplus_fused(const mv_batch_vplus_ite
     s.xjac = 1.0 / (double)it.n_cubes;  // vflowplus.py:139
     s.xdeltajac = 1.0;
     const uint32_t draw = (uint32_t)draws[tile.item];
-    // this wave's run: the tile's trips split evenly over the waves
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t trips = (end - first + 63) >> 6;
-    const int64_t a = first + (wave * trips / W) * 64;
-    const int64_t b = min(first + ((wave + 1) * trips / W) * 64, end);
-    double acc = 0.0, acc2 = 0.0;
     double* cr = ress + it.cube_offset;
     double* cr2 = ress2 + it.cube_offset;
     if constexpr (DSPEC > 0) {
       if (it.train)
-        vplus_tile_body<MIXED, FAM, true, PAIRS, DSPEC>(it, s, draw, st, a, b, tab, tw, hist, cr, cr2, acc, acc2);
+        vplus_tile_body<MIXED, FAM, true, PAIRS, DSPEC>(it, s, draw, st, a, b, c0, tab, hist, cr, cr2);
       else
-        vplus_tile_body<MIXED, FAM, false, PAIRS, DSPEC>(it, s, draw, st, a, b, tab, tw, hist, cr, cr2, acc, acc2);
+        vplus_tile_body<MIXED, FAM, false, PAIRS, DSPEC>(it, s, draw, st, a, b, c0, tab, hist, cr, cr2);
     } else {
       constexpr auto dims = std::make_integer_sequence<int, MV_FUSED_MAX_DIM>{};
       if (it.train)
-        vplus_tile_dispatch<MIXED, FAM, true, PAIRS>(dims, d, it, s, draw, st, a, b, tab, tw, hist, cr, cr2, acc,
-                                                     acc2);
+        vplus_tile_dispatch<MIXED, FAM, true, PAIRS>(dims, d, it, s, draw, st, a, b, c0, tab, hist, cr, cr2);
       else
-        vplus_tile_dispatch<MIXED, FAM, false, PAIRS>(dims, d, it, s, draw, st, a, b, tab, tw, hist, cr, cr2, acc,
-                                                      acc2);
+        vplus_tile_dispatch<MIXED, FAM, false, PAIRS>(dims, d, it, s, draw, st, a, b, c0, tab, hist, cr, cr2);
     }
     // histogram bins into the item's row (its sum columns stay unused: the
     // VEGAS+ sums are per cube)
     if (it.train) {
       if (PAIRS)
-        finish_pairs<BS, false>(acc, acc2, hist, d, rows + it.row_offset);
+        finish_pairs<BS, false>(0.0, 0.0, hist, d, rows + it.row_offset);
       else
-        finish_row<true, false>(acc, acc2, hist, nb, rows + it.row_offset);
+        finish_row<true, false>(0.0, 0.0, hist, nb, rows + it.row_offset);
     }
   }
 }
@@ -160,18 +142,29 @@ using BatchVplusKernel = void (*)(const mv_batch_vplus_item*, const mv_batch_til
                                   const double*, const int32_t*, const int32_t*, double*, double*, double*,
                                   int);
 
-template <bool MIXED, int FAM, bool PAIRS, int... Ds>
+template <bool MIXED, int FAM, bool PAIRS, int D0, int... Ds>
 constexpr std::array<BatchVplusKernel, sizeof...(Ds)> batch_vplus_table(std::integer_sequence<int, Ds...>) {
-  return {&batch_vplus_fused<MIXED, FAM, PAIRS, PAIRS ? kPairBlock : kBlock, Ds + 1>...};
+  return {&batch_vplus_fused<MIXED, FAM, PAIRS, PAIRS ? kPairBlock : kBlock, Ds + D0>...};
 }
 
 // The kernel for (family, histogram form): compiled for n_dim ``dspec``
 // (1..MV_FUSED_MAX_DIM), or choosing the body per tile (dspec 0).
 template <bool MIXED, int FAM, bool PAIRS>
 BatchVplusKernel batch_vplus_family(int dspec) {
-  static constexpr auto table =
-      batch_vplus_table<MIXED, FAM, PAIRS>(std::make_integer_sequence<int, MV_FUSED_MAX_DIM>{});
-  if (dspec >= 1 && dspec <= MV_FUSED_MAX_DIM) return table[dspec - 1];
+  // pair launches hold n_dim kPairMinDim..kPairMaxDim only, and on gfx950 the
+  // others come to per-wave launches of one n_dim only outside that range
+  if constexpr (PAIRS) {
+    static constexpr auto table = batch_vplus_table<MIXED, FAM, true, kPairMinDim>(
+        std::make_integer_sequence<int, kPairMaxDim - kPairMinDim + 1>{});
+    if (dspec >= kPairMinDim && dspec <= kPairMaxDim) return table[dspec - kPairMinDim];
+  } else {
+    static constexpr auto low =
+        batch_vplus_table<MIXED, FAM, false, 1>(std::make_integer_sequence<int, kPairMinDim - 1>{});
+    static constexpr auto high = batch_vplus_table<MIXED, FAM, false, kPairMaxDim + 1>(
+        std::make_integer_sequence<int, MV_FUSED_MAX_DIM - kPairMaxDim>{});
+    if (dspec >= 1 && dspec < kPairMinDim) return low[dspec - 1];
+    if (dspec > kPairMaxDim && dspec <= MV_FUSED_MAX_DIM) return high[dspec - kPairMaxDim - 1];
+  }
   return &batch_vplus_fused<MIXED, FAM, PAIRS, PAIRS ? kPairBlock : kBlock, 0>;
 }
 
@@ -197,7 +190,7 @@ int launch_batch_vplus_precision(const mv_batch_vplus_item* items, const mv_batc
   // pair tables whenever every tiled item can pair its dimensions and they
   // fit in a workgroup's LDS
   const int nbmax = max_dim * kBins;
-  const size_t table = MIXED ? (size_t)nbmax + (nbmax + 1) / 2 : 3 * (size_t)nbmax;
+  const size_t table = 2 * (size_t)nbmax;
   const bool pairs = min_dim >= kPairMinDim && max_dim <= kPairMaxDim &&
                      (table + (size_t)pair_cells(max_dim)) * sizeof(double) <= max_lds_per_block();
   const int dspec = min_dim == max_dim ? max_dim : 0;
@@ -214,22 +207,6 @@ int launch_batch_vplus_precision(const mv_batch_vplus_item* items, const mv_batc
   hipLaunchKernelGGL(k, dim3(blocks), dim3(bs), lds, stream, items, tiles, n_tiles, draws, grids, n_ev, offsets,
                      ress, ress2, rows, nbmax);
   return check_launch("mv_batch_vplus_fused");
-}
-
-int launch_batch_vplus_mixed(const mv_batch_vplus_item* items, const mv_batch_tile* tiles, int n_tiles, int family,
-                             int min_dim, int max_dim, const int32_t* draws, const double* grids,
-                             const int32_t* n_ev, const int32_t* offsets, double* ress, double* ress2, double* rows,
-                             int blocks, hipStream_t stream) {
-  return launch_batch_vplus_precision<true>(items, tiles, n_tiles, family, min_dim, max_dim, draws, grids, n_ev,
-                                            offsets, ress, ress2, rows, blocks, stream);
-}
-
-int launch_batch_vplus_f64(const mv_batch_vplus_item* items, const mv_batch_tile* tiles, int n_tiles, int family,
-                           int min_dim, int max_dim, const int32_t* draws, const double* grids,
-                           const int32_t* n_ev, const int32_t* offsets, double* ress, double* ress2, double* rows,
-                           int blocks, hipStream_t stream) {
-  return launch_batch_vplus_precision<false>(items, tiles, n_tiles, family, min_dim, max_dim, draws, grids, n_ev,
-                                             offsets, ress, ress2, rows, blocks, stream);
 }
 
 }  // namespace mv

@@ -249,27 +249,34 @@ __device__ __forceinline__ float Integrand<float, MV_FN_GAUSSIAN>::value() const
   return pref * __builtin_amdgcn_exp2f(-coef * 1.4426950408889634f);
 }
 
+// The mixture keeps the event's coordinates and sums one component after the
+// other: one test per component and event (n_comp is a launch-time value),
+// not one per component and dimension.
 template <typename T>
 struct Integrand<T, MV_FN_GAUSSMIX> {
   const mv_integrand* prm;
-  int nc;
-  T coef[MV_MAX_COMP];
-  __device__ explicit Integrand(const mv_integrand& p) : prm(&p), nc(p.n_comp) {}
+  int nc, n;
+  T x[MV_FUSED_MAX_DIM];
+  __device__ explicit Integrand(const mv_integrand& p) : prm(&p), nc(p.n_comp), n(0) {}
   __device__ static void fold(const mv_integrand&, int, double&, double&) {}
   __device__ static double fold_scale(const mv_integrand&, int) { return 1.0; }
-  __device__ __forceinline__ void add_folded(int j, T x) { add(j, x); }
-  __device__ __forceinline__ void begin() {
-#pragma unroll
-    for (int k = 0; k < MV_MAX_COMP; ++k) coef[k] = (T)0;
+  __device__ __forceinline__ void add_folded(int j, T v) { add(j, v); }
+  __device__ __forceinline__ void begin() { n = 0; }
+  __device__ __forceinline__ void add(int j, T v) {
+    x[j] = v;
+    n = j + 1;
   }
-  __device__ __forceinline__ void add(int j, T x) {
+  // ((x - c_k) / a_k)^2 summed over the dimensions
+  __device__ __forceinline__ T exponent(int k) const {
+    T coef = (T)0;
 #pragma unroll
-    for (int k = 0; k < MV_MAX_COMP; ++k) {
-      if (k < nc) {
-        const T t = (x - (T)prm->centre[k][j]) * (T)prm->comp[k][1];
-        coef[k] = coef[k] + t * t;
+    for (int j = 0; j < MV_FUSED_MAX_DIM; ++j) {
+      if (j < n) {
+        const T t = (x[j] - (T)prm->centre[k][j]) * (T)prm->comp[k][1];
+        coef = sizeof(T) == 8 ? (T)fma((double)t, (double)t, (double)coef) : coef + t * t;
       }
     }
+    return coef;
   }
   __device__ __forceinline__ T value() const;
 };
@@ -278,7 +285,7 @@ __device__ __forceinline__ double Integrand<double, MV_FN_GAUSSMIX>::value() con
   double f = 0.0;
 #pragma unroll
   for (int k = 0; k < MV_MAX_COMP; ++k)
-    if (k < nc) f = f + prm->comp[k][0] * (prm->comp[k][2] * exp(-coef[k]));
+    if (k < nc) f = f + prm->comp[k][0] * (prm->comp[k][2] * exp(-exponent(k)));
   return f;
 }
 template <>
@@ -288,7 +295,7 @@ __device__ __forceinline__ float Integrand<float, MV_FN_GAUSSMIX>::value() const
   for (int k = 0; k < MV_MAX_COMP; ++k)
     if (k < nc)
       f = f + (float)prm->comp[k][0] *
-                  ((float)prm->comp[k][2] * __builtin_amdgcn_exp2f(-coef[k] * 1.4426950408889634f));
+                  ((float)prm->comp[k][2] * __builtin_amdgcn_exp2f(-exponent(k) * 1.4426950408889634f));
   return f;
 }
 

@@ -31,34 +31,21 @@ __device__ __forceinline__ int find_cube(const int32_t* __restrict__ off, int n_
   return lo;
 }
 
-// Cube and n_ev of event e (lane-varying) for a wave whose events all lie in
-// cubes c0 .. c0 + 63 (c0 wave-uniform, off[c0] <= every e): a lane-parallel
-// binary lifting over the 64 offsets from c0, held one per lane and read with
-// shuffles that every lane executes. 64 consecutive events starting in cube
-// c0 lie in that window when cubes hold at least one event; a lane whose
-// event reaches the window's last cube (possible only with empty cubes past
-// it) searches the whole array instead.
-__device__ __forceinline__ int window_cube(const int32_t* __restrict__ off,
-                                          const int32_t* __restrict__ n_ev, int n_cubes, int c0, int e,
-                                          int& nev) {
+// find_cube of a wave-uniform event by the whole wave: every step probes 64
+// evenly spaced offsets at once (three loads one after the other for 1e4
+// cubes, where a binary search takes fourteen). The whole wave must be active.
+__device__ __forceinline__ int find_cube_wave(const int32_t* __restrict__ off, int n_cubes, int e) {
   const int lane = threadIdx.x & 63;
-  const int lim = min(n_cubes - c0, 64);
-  const int ok = lane < lim ? off[c0 + lane] : 0x7fffffff;
-  const int nk = lane < lim ? n_ev[c0 + lane] : 0;
-  int lo = 0;
-#pragma unroll
-  for (int stp = 32; stp >= 1; stp >>= 1) {
-    const int probe = lo + stp;  // <= 63
-    const int v = __shfl(ok, probe, 64);
-    if (probe < lim && v <= e) lo = probe;
+  int lo = 0, hi = n_cubes;  // off[lo] <= e < off[hi]
+  while (hi - lo > 1) {
+    const int stride = (hi - lo + 63) >> 6;
+    const int c = lo + lane * stride;
+    const uint64_t below = __ballot(c < hi && off[min(c, hi)] <= e);  // a prefix of the lanes, lane 0 always
+    const int i = __popcll(below) - 1;
+    hi = min(hi, lo + (i + 1) * stride);
+    lo = lo + i * stride;
   }
-  nev = __shfl(nk, lo, 64);
-  int c = c0 + lo;
-  if (lo == 63) {
-    c = find_cube(off, n_cubes, e);
-    nev = n_ev[c];
-  }
-  return c;
+  return lo;
 }
 
 // q = c / n, r = c % n for 0 <= c < 2^24 through an FP32 reciprocal and
@@ -89,20 +76,6 @@ __device__ __forceinline__ double div_by_strat(double t, double n, double y) {
   return fma(r, y, q);
 }
 
-// hypercube coordinates for a compile-time n_dim D, last dimension fastest
-// (vflowplus.py:126-128)
-template <int D>
-__device__ __forceinline__ void cube_digits_d(int cube, int n_strat, float rn, int (&h)[D]) {
-  int c = cube;
-#pragma unroll
-  for (int j = D - 1; j >= 0; --j) {
-    int q, r;
-    divmod_small(c, n_strat, rn, q, r);
-    h[j] = r;
-    c = q;
-  }
-}
-
 // Segmented suffix sum over the wave's (sorted) cube ids; the first lane of
 // each segment adds the segment total to ress / ress2 (vflowplus.py:213-214).
 __device__ __forceinline__ void segment_add(int cube, double v, double v2, double* __restrict__ ress,
@@ -129,7 +102,7 @@ __device__ __forceinline__ void segment_add(int cube, double v, double v2, doubl
 
 
 
-// The fused VEGAS+ producer (vplus_fused.hip), compiled per (integrand
+// The fused VEGAS+ producer (vplus_kernel.hpp), compiled per (integrand
 // family, train, n_dim, injected draws) for 1 <= n_dim <= MV_FUSED_MAX_DIM,
 // one launcher per precision. Return the workgroups launched or a negative
 // error.
@@ -140,7 +113,7 @@ int launch_vplus_fused_f64(int family, bool train, const StepK& k, const StrataK
                            const mv_integrand& fn, const double* grid, double* ress, double* ress2,
                            const RowsK& R, hipStream_t s);
 
-// The batched VEGAS+ producer (batch_vplus.hip) of one precision: 0 or a
+// The batched VEGAS+ producer (batch_vplus.hpp) of one precision: 0 or a
 // negative status.
 int launch_batch_vplus_mixed(const mv_batch_vplus_item* items, const mv_batch_tile* tiles, int n_tiles, int family,
                              int min_dim, int max_dim, const int32_t* draws, const double* grids,
