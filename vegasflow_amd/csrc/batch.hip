@@ -244,12 +244,14 @@ __global__ __launch_bounds__(64) void batch_finalize_kernel(const mv_batch_item*
     return;
   }
   const int64_t c = 2 + (int64_t)dim * kBins + t;
+  double* div = grids + it.grid_offset + (int64_t)dim * (kBins + 1);
+  const double edge = t <= kBins ? div[t] : 0.0;
   if (t < kBins) {
     hb[t] = row[c];
     row[c] = 0.0;
   }
   __syncthreads();
-  if (it.train && wave_hist_finite(hb)) refine_wave(hb, grids + it.grid_offset + (int64_t)dim * (kBins + 1));
+  if (it.train && wave_hist_finite(hb)) refine_wave(hb, edge, div);
 }
 
 }  // namespace mv

@@ -10,18 +10,22 @@ namespace mv {
 // Lanes 0..49 own a bin, lanes 0..50 an edge. The reference's 49 serial cuts
 // (vflow.py:194-207) are computed independently, lane k making cut k: the
 // serial loop stops in the first bin n whose running weight reaches k * ave,
-// with bw = cumsum(wei)[n] - k * ave left over, so lane k finds n, the count
-// of prefix sums below k * ave (a binary search over the non-decreasing
-// prefix sums, held one per lane), and interpolates as the reference does,
-// prev = 0.0 (not div[0]) for n = 0 included. Only the rounding of bw differs
-// from the serial accumulation (a few ulp of sum(wei)). n is capped at the
-// last bin; the reference has no guard there. The wave runs alone on its CU,
-// so its instruction latency is the kernel's time: the weight
-// (1 - r)/(log(sum) - log(s))^1.5 is taken as aux * sqrt(aux) with one log of
-// sum / s, equal to the reference's pow and two logs to a few ulp.
-__device__ inline void refine_wave(const double* h /* LDS, 50 */, double* __restrict__ div /* 51 */) {
+// with bw = cumsum(wei)[n] - k * ave left over, so lane k needs n, the count
+// of prefix sums below k * ave, and interpolates as the reference does,
+// prev = 0.0 (not div[0]) for n = 0 included. Lane b counts the cuts that its
+// prefix sum reaches (one quotient, put right by comparing the products the
+// definition names), the first cut of every bin that holds one gets the bin by
+// a lane scatter, and each cut takes that of the nearest such lane below it:
+// three lane moves, one after the other, instead of a binary search's six
+// of 64 bits. Only the rounding of bw differs from the serial accumulation (a
+// few ulp of sum(wei)). n is capped at the last bin; the reference has no
+// guard there. The wave runs alone on its CU, so its instruction latency is
+// the kernel's time: the weight (1 - r)/(log(sum) - log(s))^1.5 is taken as
+// aux * sqrt(aux) with one log of sum / s, equal to the reference's pow and
+// two logs to a few ulp, and the caller loads ``edge`` = div[lane] (lanes
+// 0..50) early, beside its own loads.
+__device__ inline void refine_wave(const double* h /* LDS, 50 */, double edge, double* __restrict__ div /* 51 */) {
   const int lane = threadIdx.x & 63;
-  const double edge = lane <= kBins ? div[lane] : 0.0;
   double s = 0.0;
   if (lane < kBins) {
     const double r = h[lane];
@@ -42,16 +46,23 @@ __device__ inline void refine_wave(const double* h /* LDS, 50 */, double* __rest
   // inclusive prefix sums of the weights (lanes >= 50 hold 0)
   const double c = wave_inclusive_scan(wei);
   const double target = (double)lane * ave;  // cut k = lane
-  // n = #{b < 50 : c_b < target}: c is non-decreasing over lanes 0..63 (lanes
-  // >= 50 repeat the total), so binary lifting over lanes; every lane runs
-  // every shuffle
-  int n = 0;
-#pragma unroll
-  for (int stp = 32; stp >= 1; stp >>= 1) {
-    const double v = __shfl(c, n + stp - 1, 64);  // c_(n + stp - 1), index <= 62
-    if (n + stp <= kBins && v < target) n += stp;
-  }
-  if (n > kBins - 1) n = kBins - 1;
+  // reached = #{k in 1..49 : k ave <= c_b} of lane b (lanes >= 50 repeat the
+  // total); the products k ave are non-decreasing in k, so c_b < k ave exactly
+  // where reached < k
+  int reached = min(max((int)(c / ave), 0), kBins - 1);
+  if ((double)reached * ave > c) --reached;
+  if (reached < kBins - 1 && (double)(reached + 1) * ave <= c) ++reached;
+  const int up = __shfl_up(reached, 1, 64);  // every lane runs every move
+  const int below = lane > 0 ? up : 0;
+  // lanes reached_(b-1) + 1 .. reached_b hold the cuts that fall in bin b
+  const bool holds = lane < kBins && reached > below;
+  const int bin1 = __builtin_amdgcn_ds_permute(holds ? (below + 1) << 2 : 0, holds ? lane + 1 : 0);  // bin + 1
+  const uint64_t starts = __ballot(bin1 != 0) & ~1ull;  // lane 0 is no cut
+  const uint64_t upto = starts & (~0ull >> (63 - lane));
+  int n = __shfl(bin1, upto ? 63 - __builtin_clzll(upto) : 0, 64) - 1;
+  // cuts past the last prefix sum (rounding): the last bin
+  if (lane > __builtin_amdgcn_readlane(reached, kBins - 1)) n = kBins - 1;
+  if (n < 0) n = 0;  // lane 0, which is no cut
   // every shuffle runs on the whole wave (a lane-gather from an inactive
   // lane reads 0); the n == 0 case is selected afterwards
   const double cn = __shfl(c, n, 64);
@@ -115,31 +126,47 @@ __device__ __forceinline__ bool wave_hist_finite(const double* hb) {
   return !__any(bad);
 }
 
-// Sum column c of the (at most MV_ROWS) group rows in order and zero it for
-// the next producer. All loads are issued before the first store so that
-// they are in flight together instead of one memory latency per row.
-__device__ __forceinline__ double take_column(double* __restrict__ P, int64_t stride, int nrows,
+// Sum column c of the group rows first .. first + N - 1 (those below nrows) in
+// order and zero it for the next producer. All loads are issued before the
+// first store so that they are in flight together instead of one memory
+// latency per row.
+template <int N>
+__device__ __forceinline__ double take_column(double* __restrict__ P, int64_t stride, int nrows, int first,
                                               int64_t c) {
-  double v[MV_ROWS];
+  double v[N];
 #pragma unroll
-  for (int r = 0; r < MV_ROWS; ++r) v[r] = r < nrows ? P[(int64_t)r * stride + c] : 0.0;
+  for (int r = 0; r < N; ++r) v[r] = first + r < nrows ? P[(int64_t)(first + r) * stride + c] : 0.0;
   double a = v[0];
 #pragma unroll
-  for (int r = 1; r < MV_ROWS; ++r)
-    if (r < nrows) a += v[r];
+  for (int r = 1; r < N; ++r) a += v[r];
 #pragma unroll
-  for (int r = 0; r < MV_ROWS; ++r)
-    if (r < nrows) P[(int64_t)r * stride + c] = 0.0;
+  for (int r = 0; r < N; ++r)
+    if (first + r < nrows) P[(int64_t)(first + r) * stride + c] = 0.0;
   return a;
 }
 
-// Sums and sigma from the group rows (vflow.py:432-442): thread v < 2 n_out
-// takes column v.
+// Sums and sigma from the group rows (vflow.py:432-442). 32 lanes take a
+// column, one row each, so that every value is in flight at once, and add
+// it within the half wave (a fixed order).
 __device__ inline void finalize_sums_block(const FzK& z, double* __restrict__ P, int64_t stride,
                                            int nrows, double* __restrict__ out) {
+  static_assert(MV_ROWS == 32, "a half wave holds a column");
   __shared__ double red[2 * MV_MAX_OUT];
   const int t = threadIdx.x;
-  if (t < 2 * z.n_out) red[t] = take_column(P, stride, nrows, t);
+  for (int i = t; i < 2 * z.n_out * MV_ROWS; i += kBlock) {  // whole waves: a multiple of 64
+    const int row = i & (MV_ROWS - 1), col = i / MV_ROWS;
+    double v = 0.0;
+    if (row < nrows) {
+      v = P[(int64_t)row * stride + col];
+      P[(int64_t)row * stride + col] = 0.0;
+    }
+    v += dpp_f64<0xB1, 0xF, true>(v);   // quad_perm [1, 0, 3, 2]
+    v += dpp_f64<0x4E, 0xF, true>(v);   // quad_perm [2, 3, 0, 1]
+    v += dpp_f64<0x124, 0xF, true>(v);  // row_ror 4
+    v += dpp_f64<0x128, 0xF, true>(v);  // row_ror 8
+    v += dpp_f64<0x142, 0xA>(v);        // row_bcast 15 into rows 1 and 3
+    if (row == MV_ROWS - 1) red[col] = v;
+  }
   __syncthreads();
   if (t < z.n_out) {
     const double N = z.n_events;
@@ -163,15 +190,23 @@ __device__ inline void finalize_sums_block(const FzK& z, double* __restrict__ P,
 __device__ inline void hist_refine_block(const FzK& z, double* __restrict__ P, int64_t stride,
                                          int nrows, int j, double* __restrict__ grid,
                                          double* __restrict__ hist_out) {
+  // four waves take eight rows each; the edges are loaded beside them
+  constexpr int W = 4, N = MV_ROWS / W;
+  __shared__ double part[W][kBins];
   __shared__ double hb[kBins];
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  double edge = 0.0;
+  if (z.refine && t <= kBins) edge = grid[j * (kBins + 1) + t];
+  if (wave < W && lane < kBins)
+    part[wave][lane] = take_column<N>(P, stride, nrows, wave * N, 2 * z.n_out + j * kBins + lane);
+  __syncthreads();
   if (t < kBins) {
-    const double a = take_column(P, stride, nrows, 2 * z.n_out + j * kBins + t);
+    const double a = ((part[0][t] + part[1][t]) + part[2][t]) + part[3][t];
     hb[t] = a;
     if (hist_out) hist_out[j * kBins + t] = a;
   }
   __syncthreads();
-  if (z.refine && t < 64 && wave_hist_finite(hb)) refine_wave(hb, grid + j * (kBins + 1));
+  if (z.refine && t < 64 && wave_hist_finite(hb)) refine_wave(hb, edge, grid + j * (kBins + 1));
 }
 
 }  // namespace mv

@@ -448,9 +448,10 @@ __global__ __launch_bounds__(64) void refine_kernel(const double* __restrict__ h
                                                     double* __restrict__ grid) {
   __shared__ double hb[kBins];
   const int j = blockIdx.x, t = threadIdx.x;
+  const double edge = t <= kBins ? grid[j * (kBins + 1) + t] : 0.0;
   if (t < kBins) hb[t] = hist[j * hstride + t];
   __syncthreads();
-  if (wave_hist_finite(hb)) refine_wave(hb, grid + j * (kBins + 1));
+  if (wave_hist_finite(hb)) refine_wave(hb, edge, grid + j * (kBins + 1));
 }
 
 // ---------------------------------------------------------------------------

@@ -141,8 +141,7 @@ __global__ __launch_bounds__(kBlock) void vplus_digest(StepK s, StrataK st, cons
 }
 
 // ---------------------------------------------------------------------------
-// iteration end over the cubes (vflowplus.py:222-242 + 153-163), one
-// workgroup of 1024 threads; thread t owns a contiguous chunk of cubes.
+// iteration end over the cubes (vflowplus.py:222-242 + 153-163)
 // ---------------------------------------------------------------------------
 // VEGAS+ iteration end over the cubes, in three launches of kBlock-thread
 // workgroups with one thread per cube (coalesced, spread over the device):
@@ -184,13 +183,13 @@ __device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* tota
 // variance max(var, 0)^(beta/2), left in ress2 for part 2; per workgroup the
 // partial sums of ress, max(var, 0) / (n_ev - 1) and the damped variances.
 // The bodies of the three kernels take the workgroup's chunk ``b`` of cubes
-// explicitly, so that the batched iteration end (batch_vplus.hip) runs them
+// explicitly, so that the batched iteration end runs them
 // for many integrals in one launch each.
 __device__ inline void cube_stats_body(int b, int n_cubes, const int32_t* __restrict__ n_ev,
                                        const double* __restrict__ ress, double* __restrict__ ress2,
                                        int adaptive, double beta, double* __restrict__ out,
                                        double* __restrict__ arr_var_out) {
-  __shared__ double part[kWaves];
+  __shared__ double part[3][kWaves];
   const int c = b * kBlock + threadIdx.x;
   double rs = 0.0, s2 = 0.0, dl = 0.0;
   if (c < n_cubes) {
@@ -205,14 +204,21 @@ __device__ inline void cube_stats_body(int b, int n_cubes, const int32_t* __rest
       ress2[c] = dl;
     }
   }
-  rs = block_sum(rs, part);
-  s2 = block_sum(s2, part);
-  dl = block_sum(dl, part);
-  if (threadIdx.x == 0) {
-    double* o = out + 3 + 3 * (int64_t)b;
-    o[0] = rs;
-    o[1] = s2;
-    o[2] = dl;
+  rs = wave_sum(rs);
+  s2 = wave_sum(s2);
+  dl = wave_sum(dl);
+  if ((threadIdx.x & 63) == 0) {
+    const int w = threadIdx.x >> 6;
+    part[0][w] = rs;
+    part[1][w] = s2;
+    part[2][w] = dl;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    const double* p = part[threadIdx.x];
+    double a = p[0];
+    for (int k = 1; k < kWaves; ++k) a += p[k];
+    out[3 + 3 * (int64_t)b + threadIdx.x] = a;
   }
 }
 
@@ -224,22 +230,17 @@ __global__ __launch_bounds__(kBlock) void vplus_cube_stats(int n_cubes, const in
   cube_stats_body(blockIdx.x, n_cubes, n_ev, ress, ress2, adaptive, beta, out, arr_var_out);
 }
 
-// The partial sums of part 1 over all workgroups, in order (every workgroup
-// of parts 2 and 3 recomputes them; there are few).
+// The partial sums of part 1 over all workgroups, in a fixed order (every
+// workgroup of part 2 recomputes them; there are few): wave k < 3 takes sum k,
+// its lanes every 64th partial, added up by wave_sum.
 __device__ __forceinline__ void cube_totals(const double* __restrict__ out, int nb, double* tot) {
-  __shared__ double buf[3][kBlock];
-  double acc = 0.0;
-  for (int b0 = 0; b0 < nb; b0 += kBlock) {
-    if (b0 + (int)threadIdx.x < nb)
-      for (int k = 0; k < 3; ++k) buf[k][threadIdx.x] = out[3 + 3 * (int64_t)(b0 + threadIdx.x) + k];
-    __syncthreads();
-    if (threadIdx.x < 3) {
-      const int m = min(kBlock, nb - b0);
-      for (int i = 0; i < m; ++i) acc = (b0 + i == 0) ? buf[threadIdx.x][i] : acc + buf[threadIdx.x][i];
-    }
-    __syncthreads();
+  const int k = threadIdx.x >> 6;
+  if (k < 3) {
+    double acc = 0.0;
+    for (int b = threadIdx.x & 63; b < nb; b += 64) acc += out[3 + 3 * (int64_t)b + k];
+    acc = wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) tot[k] = acc;
   }
-  if (threadIdx.x < 3) tot[threadIdx.x] = acc;
   __syncthreads();
 }
 
@@ -401,14 +402,15 @@ __global__ __launch_bounds__(kBlock) void batch_vplus_offsets(const mv_batch_vpl
   const mv_batch_vplus_item& it = items[item];
   __shared__ double hb[kBins];
   double* row = rows + it.row_offset + 2 + (int64_t)dim * kBins;
+  double* div = grids + it.grid_offset + (int64_t)dim * (kBins + 1);
   const int t = threadIdx.x;
+  const double edge = t <= kBins ? div[t] : 0.0;
   if (t < kBins) {
     hb[t] = row[t];
     row[t] = 0.0;
   }
   __syncthreads();
-  if (it.train && t < 64 && wave_hist_finite(hb))
-    refine_wave(hb, grids + it.grid_offset + (int64_t)dim * (kBins + 1));  // vflowplus.py:239-240
+  if (it.train && t < 64 && wave_hist_finite(hb)) refine_wave(hb, edge, div);  // vflowplus.py:239-240
 }
 
 }  // namespace mv
