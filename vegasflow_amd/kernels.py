@@ -9,6 +9,7 @@ them directly (e.g. with injected draws).
 import ctypes
 import gc
 
+import numpy as np
 import torch
 
 from . import _abi
@@ -230,25 +231,52 @@ def capture_graph(body):
 
 
 class IterationCounter:
-    """Device iteration counter for replayed iterations: ``draw`` (int32 x 2)
-    holds {draw id of the next iteration, draw id of history slot 0};
-    steps read the draw id from it and the finalize kernels store {res,
-    sigma, events} of each iteration in ``history`` (float64, 3 * capacity)
-    and advance it."""
+    """Device state of replayed iterations, in one buffer so that a run reads
+    it back with one copy: ``draw`` (int32 x 2) holds {draw id of the next
+    iteration, draw id of history slot 0}; ``status`` (int32) the MV_STATUS_*
+    bits; ``out`` (float64, ``out_len``) an algorithm's own results; steps read
+    the draw id from ``draw`` and the finalize kernels store {res, sigma,
+    events} of each iteration in ``history`` (float64, 3 * capacity) and
+    advance it."""
 
-    def __init__(self, device, capacity):
-        self.draw = torch.zeros(2, dtype=torch.int32, device=device)
+    def __init__(self, device, capacity, out_len=0):
         self.capacity = int(capacity)
-        self.history = torch.zeros(3 * self.capacity, dtype=torch.float64, device=device)
+        self.out_len = int(out_len)
+        self._buffer = torch.zeros(2 + self.out_len + 3 * self.capacity, dtype=torch.float64, device=device)
+        words = self._buffer[:2].view(torch.int32)
+        self.draw = words[:2]
+        self.status = words[2:3]
+        self.out = self._buffer[2 : 2 + self.out_len]
+        self.history = self._buffer[2 + self.out_len :]
+        self._next = None    # the draw id that ``draw`` holds once the runs so far are done
+        self._slot = 0       # the history slot of that draw
+        self._clean = True   # ``status`` is zero
 
-    def start(self, draw_id):
-        """Next iteration draws ``draw_id`` and lands in history slot 0 (a
-        fill kernel on the current stream: no host-to-device copy)."""
-        self.draw.fill_(int(draw_id))
+    def start(self, draw_id, n):
+        """The next ``n`` iterations draw ``draw_id`` and on; returns the
+        history slot of the first. The counter follows by itself from one run
+        to the next, so it is set (a fill kernel on the current stream) only
+        where the draws jump or the history is full."""
+        if self._next != draw_id or self._slot + n > self.capacity:
+            self.draw.fill_(int(draw_id))
+            self._slot = 0
+        if not self._clean:
+            self.status.zero_()
+        slot = self._slot
+        self._slot += n
+        # known again once this run has read its results (``read``)
+        self._next, self._clean = None, False
+        return slot
 
-    def results(self, n):
-        """(n, 3) device view of the first n iterations' {res, sigma, events}."""
-        return self.history[: 3 * n].view(n, 3)
+    def read(self, draw_id, slot, n):
+        """The status bits, ``out`` and the (n, 3) {res, sigma, events} of
+        the iterations from history slot ``slot`` on (which start() returned
+        for ``draw_id``), on the host: one synchronising copy."""
+        first = 2 + self.out_len + 3 * slot
+        host = self._buffer[: first + 3 * n].cpu().numpy()
+        status = int(host[:2].view(np.int32)[2])
+        self._next, self._clean = draw_id + n, status == 0
+        return status, host[2 : 2 + self.out_len], host[first:].reshape(n, 3)
 
 
 # ---------------------------------------------------------------------------
@@ -423,16 +451,25 @@ def vplus_digest(step, strata, f, w, idx, seg, ress, ress2, ws):
                      _ptr(idx), _ptr(seg), _ptr(ress), _ptr(ress2), ws.partials(), _stream())
 
 
+def vplus_out_len(n_cubes):
+    return int(_abi.load().mv_vplus_out_len(int(n_cubes)))
+
+
 def vplus_finalize(n_dim, strata, n_ev, offsets, ress, ress2, adaptive, min_neval, init_calls, beta,
                    ws, n_rows, train, refine, grid, arr_var_out=None, hist_out=None, counter=None,
-                   status=None):
+                   status=None, out=None):
     """Returns a (3,) float64 tensor: res, sigma, events of the next iteration.
-    ``counter``: an IterationCounter, as in vegas_finalize."""
+    ``counter``: an IterationCounter, as in vegas_finalize. ``out``: a float64
+    tensor of vplus_out_len(n_cubes) entries to use for them."""
     _need_device(status, "status", torch.int32)
     if _recording is not None:  # raw addresses below
         _recording.keep.append(counter)
-    out = torch.empty(int(_abi.load().mv_vplus_out_len(int(strata.n_cubes))), dtype=torch.float64,
-                      device=ws.device)
+    out_len = vplus_out_len(strata.n_cubes)
+    if out is None:
+        out = torch.empty(out_len, dtype=torch.float64, device=ws.device)
+    _need_device(out, "out", torch.float64)
+    if out.numel() < out_len:
+        raise ValueError(f"out needs {out_len} entries")
     _call("mv_vplus_finalize", int(n_dim), ctypes.byref(strata), _ptr(n_ev), _ptr(offsets), _ptr(ress),
               _ptr(ress2), int(bool(adaptive)), int(min_neval), float(init_calls), float(beta),
               _ptr(ws.rows), ws.stride, int(n_rows), int(bool(train)), int(bool(refine)),

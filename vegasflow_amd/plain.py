@@ -61,7 +61,7 @@ class PlainFlow(MonteCarloFlow):
         step = self._step(n, train=False, offset=0, draw_dev=counter.draw)
         ng = kernels.plain_fused(step, self._fused, ws)
         kernels.vegas_finalize(self.n_dim, 1, False, False, n, ws, ng, counter=counter,
-                               status=self._status_word())
+                               status=counter.status)
 
     def _fused_iteration(self, inject=None):
         self._next_draw()

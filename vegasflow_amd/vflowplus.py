@@ -254,16 +254,19 @@ class VegasFlowPlus(VegasFlow):
                           draw_dev=counter.draw)
         strata = self._strata()
         ng = kernels.vplus_fused(step, strata, self._fused, self.divisions, self._ress, self._ress2, ws)
-        return kernels.vplus_finalize(self.n_dim, strata, self._n_ev, self._offsets, self._ress, self._ress2,
+        kernels.vplus_finalize(self.n_dim, strata, self._n_ev, self._offsets, self._ress, self._ress2,
                                       self._adaptive, self.min_neval_hcube, self._init_calls, BETA, ws, ng,
                                       self.train, self.train, self.divisions, counter=counter,
-                                      status=self._status_word())
+                                      status=counter.status, out=counter.out)
 
-    def _replayed_events(self, events):
+    def _counter_out_len(self):
+        return kernels.vplus_out_len(self._n_cubes)
+
+    def _replayed_events(self, events, out):
         # events of each replayed iteration, and the next iteration's count
         # from the last finalize
-        self._pending_events.extend(int(e) for e in events)
-        self._last_out = self._replay_last
+        self.events_history.extend(int(e) for e in events)
+        self._n_events = int(out[2])
 
     def _fused_iteration(self, inject=None):
         self._next_draw()
@@ -287,9 +290,9 @@ class VegasFlowPlus(VegasFlow):
         self._last_out = out
         return out[0], out[1]
 
-    def _device_extras(self, replayed):
+    def _device_extras(self):
         # the event counts still on the device, then the next iteration's
-        last = self._replay_last if replayed else self._last_out
+        last = self._last_out
         pend = [e.reshape(()) for e in self._pending_events if torch.is_tensor(e)]
         self._extras_layout = (len(pend), last is not None)
         return pend + ([last[2].reshape(())] if last is not None else [])
