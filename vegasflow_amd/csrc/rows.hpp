@@ -172,6 +172,12 @@ __device__ __forceinline__ void event_trips(const StepK& s, Body&& body) {
   if (i0 + full * step < s.n_events) body(c);
 }
 
+// Start of share g of ``trips`` split evenly over ``n`` (g = 0 .. n, n > 0): a
+// non-decreasing function with trip_of(0) = 0 and trip_of(n) = trips.
+__device__ __forceinline__ int64_t trip_of(int64_t g, int64_t trips, int64_t n) {
+  return g >= n ? trips : (int64_t)((double)g * ((double)trips / (double)n));
+}
+
 // this workgroup's group row
 __device__ __forceinline__ double* group_row(const RowsK& R) {
   return R.rows + (int64_t)(blockIdx.x % kRows) * R.stride;

@@ -20,6 +20,7 @@
 #include "fused_event.hpp"
 #include "refine.hpp"
 #include "rows.hpp"
+#include "vplus.hpp"
 
 namespace mv {
 
@@ -346,90 +347,6 @@ __global__ __launch_bounds__(kBlock) void vegas_digest(StepK s, const FT* __rest
   }
 }
 
-// Training digest of a scalar integrand with pair histograms (fused_event.hpp)
-// for 2 <= n_dim <= kPairMaxDim: one LDS add per pair of dimensions into a
-// workgroup's pair tables (LDS: pair_cells(d) doubles), so the kernel is
-// bound by its HBM reads (f, w, bins) rather than by LDS atomics. Rows of
-// bins whose length is a multiple of 4 are read four bins per load. Bins
-// are clamped to 0..49 as in vegas_digest.
-constexpr int kDigestU = 4;  // events per trip of the pair digest's word path
-
-template <typename FT, int BS>
-__global__ __launch_bounds__(BS) void vegas_digest_pairs(StepK s, const FT* __restrict__ f,
-                                                         int64_t fstride, const FT* __restrict__ w,
-                                                         int64_t wstride, const uint8_t* __restrict__ idx,
-                                                         RowsK R) {
-  extern __shared__ double H[];
-  const int d = s.n_dim;
-  const int half = pair_cells(d) / 2;
-  for (int i = threadIdx.x; i < half; i += BS) reinterpret_cast<double2*>(H)[i] = make_double2(0.0, 0.0);
-  __syncthreads();
-  const int np = (d + 1) >> 1;
-  const bool words = (d & 3) == 0 && ((uintptr_t)idx & 3u) == 0;
-  const uint32_t top = kBins - 1;
-  double acc = 0.0, acc2 = 0.0;
-  const int64_t step = (int64_t)gridDim.x * BS;
-  const int64_t i0 = spread_first_event();
-  if (words) {
-    // kDigestU events per trip, all their loads issued before the first is
-    // used: with one workgroup per CU the loop is otherwise bound by one
-    // memory latency per event. Sums are added in event order.
-    constexpr int U = kDigestU;
-    constexpr int MAXW = kPairMaxDim / 4;
-    const int nw = d >> 2;
-    for (int64_t i = i0; i < s.n_events; i += U * step) {
-      double tmp[U];
-      uint32_t v[U][MAXW];
-      bool ok[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t e = i + u * step;
-        ok[u] = e < s.n_events;
-        tmp[u] = 0.0;
-#pragma unroll
-        for (int g = 0; g < MAXW; ++g) v[u][g] = 0u;
-        if (ok[u]) {
-          tmp[u] = (double)w[e * wstride] * (double)f[e * fstride];  // vflow.py:416
-          const uint32_t* ir4 = reinterpret_cast<const uint32_t*>(idx + e * d);  // 4-aligned
-#pragma unroll
-          for (int g = 0; g < MAXW; ++g)
-            if (g < nw) v[u][g] = ir4[g];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (!ok[u]) continue;
-        const double tmp2 = tmp[u] * tmp[u];
-        acc += tmp[u];
-        acc2 += tmp2;
-#pragma unroll
-        for (int g = 0; g < MAXW; ++g) {
-          if (g < nw) {
-            const uint32_t x = v[u][g];
-            const uint32_t b0 = min(x & 0xffu, top), b1 = min((x >> 8) & 0xffu, top);
-            const uint32_t b2 = min((x >> 16) & 0xffu, top), b3 = min(x >> 24, top);
-            lds_add(&H[(2 * g) * kPairBins + b0 * kBins + b1], tmp2);
-            lds_add(&H[(2 * g + 1) * kPairBins + b2 * kBins + b3], tmp2);
-          }
-        }
-      }
-    }
-  } else {
-    for (int64_t i = i0; i < s.n_events; i += step) {
-      const double tmp = (double)w[i * wstride] * (double)f[i * fstride];  // vflow.py:416
-      const double tmp2 = tmp * tmp;
-      acc += tmp;
-      acc2 += tmp2;
-      const uint8_t* ir = idx + i * d;
-      for (int p = 0; p < np; ++p) {
-        const uint32_t b0 = min((uint32_t)ir[2 * p], top);
-        const uint32_t b1 = 2 * p + 1 < d ? min((uint32_t)ir[2 * p + 1], top) : 0u;
-        lds_add(&H[p * kPairBins + b0 * kBins + b1], tmp2);
-      }
-    }
-  }
-  finish_pairs<BS>(acc, acc2, H, d, group_row(R));
-}
 // ---------------------------------------------------------------------------
 // finalize: block 0 sums and sigma, block 1 + j dimension j (refine.hpp)
 // ---------------------------------------------------------------------------
@@ -630,6 +547,7 @@ extern "C" int mv_vegas_sample(const mv_step* step, const double* grid, void* x,
     uint8_t* io = idx ? idx + e0 * d : nullptr;
     void* xp = static_cast<char*>(x) + e0 * d * (int64_t)elem;
     void* wp = static_cast<char*>(w) + e0 * (int64_t)elem;
+    if (launch_vegas_sample(k, !f64, grid, xp, wp, io, st)) return blocks;
     if (f64) {
       if (staged) hipLaunchKernelGGL((vegas_sample<false, true>), dim3(blocks), dim3(kBlock), lds, st, k, grid, xp, wp, io);
       else hipLaunchKernelGGL((vegas_sample<false, false>), dim3(blocks), dim3(kBlock), 0, st, k, grid, xp, wp, io);
@@ -656,6 +574,7 @@ extern "C" int mv_plain_sample(const mv_step* step, void* x, void* stream) {
   for_each_counter_range(*step, elem, [&](const StepK& k, int64_t e0) {
     const int blocks = sample_blocks(k.n_events);
     void* xp = static_cast<char*>(x) + e0 * d * (int64_t)elem;
+    if (launch_plain_sample(k, !f64, xp, st)) return blocks;
     if (f64) {
       if (staged) hipLaunchKernelGGL((plain_sample<false, true>), dim3(blocks), dim3(kBlock), lds, st, k, xp);
       else hipLaunchKernelGGL((plain_sample<false, false>), dim3(blocks), dim3(kBlock), 0, st, k, xp);
@@ -687,20 +606,10 @@ extern "C" int mv_vegas_digest(const mv_step* step, const void* f, int64_t f_str
     return rc;
   const StepK k = make_stepk(*step);
   hipStream_t st = as_stream(stream);
-  const int d = step->n_dim;
-  if (step->train && n_out == 1 && d >= kPairMinDim && d <= kPairMaxDim) {
-    const size_t lds = (size_t)pair_cells(d) * sizeof(double);
-    if (lds <= max_lds_per_block()) {
-      const int b = step->precision == MV_F64
-          ? launch_producer<kPairBlock>(vegas_digest_pairs<double, kPairBlock>, step->n_events, lds, st, k,
-                                        static_cast<const double*>(f), f_stride,
-                                        static_cast<const double*>(w), w_stride, idx, R)
-          : launch_producer<kPairBlock>(vegas_digest_pairs<float, kPairBlock>, step->n_events, lds, st, k,
-                                        static_cast<const float*>(f), f_stride,
-                                        static_cast<const float*>(w), w_stride, idx, R);
-      if ((rc = check_launch("mv_vegas_digest"))) return rc;
-      return rows_used(b);
-    }
+  if (step->train && n_out == 1 && digest_pairs_takes(step->n_dim)) {
+    const int b = launch_digest_pairs(k, step->precision == MV_MIXED, f, f_stride, w, w_stride, idx, R, st);
+    if ((rc = check_launch("mv_vegas_digest"))) return rc;
+    return rows_used(b);
   }
   const int blocks = producer_blocks(step->n_events);
   const int slices = step->train ? (step->n_dim + kDigestDims - 1) / kDigestDims : 1;

@@ -467,6 +467,8 @@ extern "C" int mv_vplus_sample(const mv_step* step, const mv_strata* strata, con
   if (step->n_events >= (int64_t)1 << 31) return fail(MV_ERR_UNSUPPORTED, "mv_vplus_sample: too many events");
   const StepK k = make_stepk(*step);
   const StrataK st = make_strata(*strata);
+  if (launch_vplus_sample(k, step->precision == MV_MIXED, st, grid, x, w, idx, seg, as_stream(stream)))
+    return check_launch("mv_vplus_sample");
   int64_t b = (step->n_events + kBlock - 1) / kBlock;
   const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>(b, 8192));
   if (step->precision == MV_MIXED)
@@ -490,9 +492,15 @@ extern "C" int mv_vplus_digest(const mv_step* step, const mv_strata* strata, con
   if ((rc = make_rows(parts, mv_partial_stride(step->n_dim, 1, step->train),
                       "mv_vplus_digest", &R)))
     return rc;
-  const int blocks = producer_blocks(step->n_events);
   const StepK k = make_stepk(*step);
   const StrataK st = make_strata(*strata);
+  if (step->train && digest_pairs_takes(step->n_dim)) {
+    const int b = launch_vplus_digest_pairs(k, step->precision == MV_MIXED, st, f, w, idx, seg, ress, ress2, R,
+                                            as_stream(stream));
+    if ((rc = check_launch("mv_vplus_digest"))) return rc;
+    return rows_used(b);
+  }
+  const int blocks = producer_blocks(step->n_events);
   const size_t lds = step->train ? (size_t)kWaves * step->n_dim * kBins * sizeof(double) : 0;
   hipStream_t s = as_stream(stream);
 #define MV_VPD(FT, TR) \

@@ -99,8 +99,22 @@ __device__ __forceinline__ void segment_add(int cube, double v, double v2, doubl
   }
 }
 
+// The samplers with a compile-time n_dim (sample.hip) for Philox draws and
+// n_dim <= MV_FUSED_MAX_DIM; false, with nothing launched, for anything else.
+bool launch_plain_sample(const StepK& s, bool mixed, void* x, hipStream_t stream);
+bool launch_vegas_sample(const StepK& s, bool mixed, const double* grid, void* x, void* w, uint8_t* idx,
+                         hipStream_t stream);
+bool launch_vplus_sample(const StepK& s, bool mixed, const StrataK& st, const double* grid, void* x, void* w,
+                         uint8_t* idx, int32_t* seg, hipStream_t stream);
 
-
+// The training digests with pair histograms (digest.hip), for the n_dim that
+// digest_pairs_takes. Return the workgroups launched.
+bool digest_pairs_takes(int n_dim);
+int launch_digest_pairs(const StepK& s, bool mixed, const void* f, int64_t fstride, const void* w, int64_t wstride,
+                        const uint8_t* idx, const RowsK& R, hipStream_t stream);
+int launch_vplus_digest_pairs(const StepK& s, bool mixed, const StrataK& st, const void* f, const void* w,
+                              const uint8_t* idx, const int32_t* seg, double* ress, double* ress2, const RowsK& R,
+                              hipStream_t stream);
 
 // The fused VEGAS+ producer (vplus_kernel.hpp), compiled per (integrand
 // family, train, n_dim, injected draws) for 1 <= n_dim <= MV_FUSED_MAX_DIM,

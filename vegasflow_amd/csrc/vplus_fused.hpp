@@ -217,12 +217,6 @@ __device__ __forceinline__ double segment_scan(double v, int seg) {
   return v;
 }
 
-// Start of share g of ``trips`` split evenly over ``n`` (g = 0 .. n, n > 0): a
-// non-decreasing function with trip_of(0) = 0 and trip_of(n) = trips.
-__device__ __forceinline__ int64_t trip_of(int64_t g, int64_t trips, int64_t n) {
-  return g >= n ? trips : (int64_t)((double)g * ((double)trips / (double)n));
-}
-
 // The wave's run of events first .. end - 1, 64 per trip, into the per-cube
 // sums ress, ress2 (vflowplus.py:213-214) and the histograms. ``c0``: the
 // cube of event ``first`` (find_cube_wave). Measured on the two-Gaussian
