@@ -47,7 +47,7 @@ __global__ __launch_bounds__(kPairBlock) void vegas_fused_pairs(StepK s, mv_inte
       acc2 += tmp * tmp;
     }
   } else {
-    event_trips<kPairBlock>(s, [&](uint32_t c) {
+    event_trips<kPairBlock, (D > 6)>(s, [&](uint32_t c) {
       const double tmp = event_mixed_pairs<FAM, false>(F, c, s.ev_hi, draw, s.key, D, tab, cs, H, nullptr,
                                                        wscale);
       acc += tmp;

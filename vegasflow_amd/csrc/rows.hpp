@@ -151,13 +151,51 @@ __device__ __forceinline__ int64_t spread_first_event() {
   return ((int64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x) * 64 + (threadIdx.x & 63);
 }
 
+// for (t = first; t < end; t += next) body(t). PACED: with the wave's issue
+// priority falling from 3 to 0 as its trips get done, at a half, seven eighths
+// and thirty-one thirty-seconds of them. Otherwise the oldest wave of a SIMD
+// goes first: with four equal waves per SIMD they end at 25, 32, 39 and 45 us
+// (mixed pair kernel, d = 8, 1e7 events), and the last one runs alone, its LDS
+// latencies uncovered. Paced, a wave that is behind goes first and all end
+// together: 46.8 -> 45.0 us. For kernels with one workgroup of 16 waves per CU
+// whose waves wait for the LDS; the FP64 pair kernel, which its arithmetic
+// fills also from one wave, gains nothing (86.8 -> 86.2 us), and with two
+// workgroups per CU it costs: the second one stands still until the first is
+// nearly done (mixed d = 4 25.5 -> 26.9 us, FP64 49.8 -> 53.9 us).
+template <bool PACED, typename I, typename Body>
+__device__ __forceinline__ void paced_trips(I first, I end, I next, Body&& body) {
+  I t = first;
+  if constexpr (!PACED) {
+    for (; t < end; t += next) body(t);
+  } else {
+    const I todo = end > first ? end - first : 0;
+#pragma unroll 1
+    for (int phase = 0; phase < 4; ++phase) {
+      I until = end;
+      if (phase == 0) {
+        __builtin_amdgcn_s_setprio(3);
+        until = end - (todo >> 1);
+      } else if (phase == 1) {
+        __builtin_amdgcn_s_setprio(2);
+        until = end - (todo >> 3);
+      } else if (phase == 2) {
+        __builtin_amdgcn_s_setprio(1);
+        until = end - (todo >> 5);
+      } else {
+        __builtin_amdgcn_s_setprio(0);
+      }
+      for (; t < until; t += next) body(t);
+    }
+  }
+}
+
 // Runs ``body(counter word)`` for every event of this thread (the events of
 // spread_first_event, BS-thread workgroups). The wave's trips in which all 64
 // lanes have an event are counted on the scalar unit and run without a
 // per-lane test; at most one trip with a per-lane test follows. The Philox
 // counter word advances by the step (mod 2^32) as the 64-bit event index
 // would.
-template <int BS, typename Body>
+template <int BS, bool PACED = false, typename Body>
 __device__ __forceinline__ void event_trips(const StepK& s, Body&& body) {
   const int64_t step = (int64_t)gridDim.x * BS;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -165,10 +203,10 @@ __device__ __forceinline__ void event_trips(const StepK& s, Body&& body) {
   const int64_t i0 = w0 + (threadIdx.x & 63);
   const int64_t full = s.n_events - 64 - w0 >= 0 ? (s.n_events - 64 - w0) / step + 1 : 0;
   uint32_t c = s.ev_lo + (uint32_t)i0;
-  for (int64_t t = 0; t < full; ++t) {
+  paced_trips<PACED, int64_t>(0, full, 1, [&](int64_t) {
     body(c);
     c += (uint32_t)step;
-  }
+  });
   if (i0 + full * step < s.n_events) body(c);
 }
 
