@@ -151,6 +151,25 @@ __device__ __forceinline__ int64_t spread_first_event() {
   return ((int64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x) * 64 + (threadIdx.x & 63);
 }
 
+// Sets the wave's issue priority for ``left`` of ``todo`` trips to go and
+// returns how many may be left at the next change (0: none follows).
+__device__ __forceinline__ int pace(int todo, int left) {
+  if (left > todo >> 1) {
+    __builtin_amdgcn_s_setprio(3);
+    return todo >> 1;
+  }
+  if (left > todo >> 3) {
+    __builtin_amdgcn_s_setprio(2);
+    return todo >> 3;
+  }
+  if (left > todo >> 5) {
+    __builtin_amdgcn_s_setprio(1);
+    return todo >> 5;
+  }
+  __builtin_amdgcn_s_setprio(0);
+  return 0;
+}
+
 // for (t = first; t < end; t += next) body(t). PACED: with the wave's issue
 // priority falling from 3 to 0 as its trips get done, at a half, seven eighths
 // and thirty-one thirty-seconds of them. Otherwise the oldest wave of a SIMD

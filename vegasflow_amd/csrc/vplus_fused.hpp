@@ -244,6 +244,11 @@ __device__ __forceinline__ void vplus_run(Integrand<T, FAM>& F, const StepK& s, 
   double hv = 0.0, hv2 = 0.0;
   int based = -1;  // the cube that every lane's base and rn belong to, or -1
   double base[D], rn = 0.0;
+  // one workgroup of 16 waves per CU (paced_trips): 95.1 -> 87.8 us mixed, 2e7
+  // events, 19.5 -> 18.7 us FP64, 1e6 events
+  constexpr bool PACED = PAIRS;
+  int left = (int)((end - first + 63) >> 6), change = left;
+  const int todo = left;
   // pieces of the run that do not cross a multiple of 2^32 in the event
   // counter (one, unless the run crosses it)
   for (int64_t from = first, to; from < end; from = to) {
@@ -251,6 +256,7 @@ __device__ __forceinline__ void vplus_run(Integrand<T, FAM>& F, const StepK& s, 
     to = min(end, from + (int64_t)((1ull << 32) - (ge & 0xffffffffull)));
     const uint32_t ev_hi = (uint32_t)(ge >> 32);
     for (int64_t trip = from; trip < to; trip += 64) {
+      if (PACED && left-- <= change) change = pace(todo, left + 1);
       const int b = (int)trip;                          // events of an iteration < 2^31
       const int n_live = (int)min((int64_t)64, to - trip);
       const int last = b + (n_live - 1);
