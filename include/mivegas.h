@@ -329,8 +329,9 @@ int mv_batch_fused(const mv_batch_item* items, int32_t n_items, const mv_batch_t
 /* As mv_batch_fused in MV_MIXED, with the histograms of training items kept
  * as pair tables (dimensions 2p and 2p + 1 share a 50 x 50 table: one LDS
  * atomic per pair of dimensions) in 1024-thread workgroups; frozen items
- * run as in mv_batch_fused. Requires max_dim <= 14. ``blocks`` persistent
- * workgroups of 1024 threads; mv_batch_pairs_blocks(family, max_dim) is the
+ * run as in mv_batch_fused. Requires max_dim <= 14. The tiles are split
+ * evenly over ``blocks`` persistent workgroups of 1024 threads, which cut them
+ * and join those that follow each other in one item; mv_batch_pairs_blocks(family, max_dim) is the
  * number resident on the current device at once (0: unsupported). No
  * counterpart in the reference (batching is an addition). */
 int mv_batch_fused_pairs(const mv_batch_item* items, int32_t n_items, const mv_batch_tile* tiles,

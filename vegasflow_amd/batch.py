@@ -3,9 +3,8 @@
 Each item is a VegasFlow integral (built-in integrand, n_dim <= 16, its own
 event count and Philox seed). One iteration round is one persistent launch
 of ``mv_batch_fused`` (or the pair-histogram kernel, ``mv_batch_fused_pairs``
-or ``mv_batch_fused_pairs_f64``) per integrand family present (workgroups
-stride over tiles of consecutive events of one item) plus one
-``mv_batch_finalize``
+or ``mv_batch_fused_pairs_f64``) per integrand family present (over tiles of
+consecutive events of one item) plus one ``mv_batch_finalize``
 (sums, sigma, running weighted average, history, grid refinement), with all
 state resident on the device. Item i draws exactly what
 ``VegasFlow(n_dim_i, n_events_i, seed=seed_i)`` would, so its results equal a
@@ -114,12 +113,14 @@ class BatchVegas:
         self.events_per_tile = int(events_per_tile)
         self.pairs = bool(pair_histograms)
         self.blocks = int(blocks_per_cu or autotune.BLOCKS_PER_CU[-1]) * self._cus
-        self._launches = self._tile_launches(self.events_per_tile)
+        self._launches = self._tile_launches(self.events_per_tile, self.pairs)
         self._pair_blocks = self._pair_launch_blocks(self._launches) if self.pairs else {}
 
     # ------------------------------------------------------------ tiling
-    def _tile_launches(self, events_per_tile):
-        """One launch per family present: (family, tiles tensor, n_tiles, max_dim)."""
+    def _tile_launches(self, events_per_tile, pairs):
+        """One launch per family present: (family, tiles tensor, n_tiles, max_dim).
+        The pair kernel splits the list itself and joins tiles that follow
+        each other in one item: they stay in order."""
         by_family = {}
         for i, (fn, d, n, _) in enumerate(self.specs):
             by_family.setdefault(fn.family, []).append(i)
@@ -130,8 +131,8 @@ class BatchVegas:
                 n = self.specs[i][2]
                 for first in range(0, n, events_per_tile):
                     tiles.append((i, min(events_per_tile, n - first), first))
-            # heaviest tiles (most dimensions, full tiles) first
-            tiles.sort(key=lambda t: (-self.specs[t[0]][1] * t[1], t[0], t[2]))
+            if not pairs:  # heaviest tiles (most dimensions, full tiles) first
+                tiles.sort(key=lambda t: (-self.specs[t[0]][1] * t[1], t[0], t[2]))
             arr = (_abi.BatchTile * len(tiles))()
             for k, (i, c, f) in enumerate(tiles):
                 arr[k].item, arr[k].count, arr[k].first = i, c, f
@@ -168,7 +169,7 @@ class BatchVegas:
 
         def measure(cand):
             ept, bpc, pairs = cand
-            launches = self._tile_launches(ept)
+            launches = self._tile_launches(ept, pairs)
             pair_blocks = self._pair_launch_blocks(launches) if pairs else {}
             bpc = bpc or autotune.BLOCKS_PER_CU[-1]
 

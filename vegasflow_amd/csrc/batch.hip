@@ -1,14 +1,25 @@
 // batch.hip - many independent VegasFlow integrals in one persistent launch.
 //
 // The events of every item of an iteration round are cut into tiles of
-// consecutive events of one item; ``blocks`` workgroups stride over the tile
-// list. A tile loads its item's map table into LDS, runs the same per-event
-// body as the single-integral fused kernels (fused_event.hpp) and adds its
-// sums and histogram into the item's row with FP64 atomics. The finalize
-// kernel gives one wave per (item, sums) and per (item, dimension) job.
-// Grids, rows, per-item draw counters, running weighted averages and the
-// per-iteration history all stay on the device, so a round can be replayed
-// from a captured HIP graph: nothing in it depends on host values.
+// consecutive events of one item. batch_fused: ``blocks`` workgroups stride
+// over the tile list. batch_fused_pairs: the list is split evenly over the
+// workgroups (tiles.hpp). A tile or span loads its item's map table into LDS,
+// runs the same per-event body as the single-integral fused kernels
+// (fused_event.hpp) and adds its sums and histogram into the item's row with
+// FP64 atomics. The finalize kernel gives one wave per (item, sums) and per
+// (item, dimension) job. Grids, rows, per-item draw counters, running weighted
+// averages and the per-iteration history all stay on the device, so a round
+// can be replayed from a captured HIP graph: nothing in it depends on host
+// values.
+//
+// batch_fused_pairs is bound like the single pair kernel (VALU and LDS of one
+// workgroup of 16 waves per CU) plus 17 us per launch (split 6, table and
+// cleared histograms 2, marginals and row, launch). 256 Gaussians of d 2..12
+// and 1e4..1e6 events, 5.3e7 events per round: 270 us with whole tiles dealt
+// out in turn and the prologue and epilogue compiled per n_dim around the
+// event loop (table reads issued one by one for want of scalar registers),
+// 251 us with the split, 238 us with paced waves, 231 us with measured costs;
+// the single kernel's rates for the same events come to 185 us.
 #include <algorithm>
 #include <type_traits>
 
@@ -17,6 +28,7 @@
 #include "fused_event.hpp"
 #include "refine.hpp"
 #include "rows.hpp"
+#include "tiles.hpp"
 
 namespace mv {
 
@@ -102,109 +114,136 @@ __global__ __launch_bounds__(kBlock) void batch_fused(const mv_batch_item* __res
   }
 }
 
-// Tiles with pair histograms (fused_event.hpp), BS threads. LDS = the map
-// table (mixed: nbmax float2; FP64: nbmax double2), then
-// pair_cells(max_dim) doubles. Training items add one LDS atomic per pair of
-// dimensions; frozen items run the plain event body of their precision.
-template <int FAM, int BS, bool MIXED, int D = 0>
-__device__ __forceinline__ void batch_tile_pairs(const mv_batch_item& it, const mv_batch_tile& tile,
-                                                 uint32_t draw, const double* __restrict__ grids,
-                                                 double* __restrict__ rows, double* smem, int nbmax) {
-  const int d = D ? D : it.n_dim;  // D > 0: compiled for that n_dim (straight-line event body)
-  // 16-byte aligned: nbmax * 8 is a multiple of 400
-  double* H = smem + (MIXED ? nbmax : 2 * nbmax);
-  __syncthreads();  // the previous tile is done with the LDS
+// ``body(k)`` for the events k = 0 .. count - 1 of a span, 64 consecutive ones
+// per wave and trip; only the last, partial trip has a per-lane test.
+template <int BS, bool PACED, typename Body>
+__device__ __forceinline__ void span_trips(int count, Body&& body) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int full = count >> 6;
+  uint32_t k = (uint32_t)(wave * 64 + lane);
+  paced_trips<PACED, int>(wave, full, BS / 64, [&](int) {
+    body(k);
+    k += BS;
+  });
+  if (full % (BS / 64) == wave && k < (uint32_t)count) body(k);
+}
+
+// The events of a span for D = n_dim (0: it.n_dim, chosen at run time): sums
+// into acc, acc2 and, for training items, the pair tables. Only this part is
+// compiled per n_dim: with the map table and the row inside it, the addresses
+// and masks of all its copies were hoisted out of the loop over spans, which
+// left so few scalar registers that the table reads were issued one by one.
+template <int FAM, int BS, bool MIXED, int D>
+__device__ __forceinline__ void batch_span_events(const mv_batch_item& it, const mv_batch_tile& tile, uint32_t draw,
+                                                  double* smem, double& acc, double& acc2) {
+  using T = typename std::conditional<MIXED, float, double>::type;
+  using T2 = typename std::conditional<MIXED, float2, double2>::type;
+  const int d = D ? D : it.n_dim;
+  const int groups = (d + 3) / 4;
   const Key key{(uint32_t)(it.seed & 0xffffffffu), (uint32_t)(it.seed >> 32)};
   const double wscale = 1.0 / (double)it.n_events;  // xjac, monte_carlo.py:224-227
   // a tile never crosses a multiple of 2^32 events: uniform high counter word
   const uint32_t lo0 = (uint32_t)((uint64_t)tile.first & 0xffffffffu);
   const uint32_t hi = (uint32_t)((uint64_t)tile.first >> 32);
-  const int groups = (d + 3) / 4;
+  const T2* tab = reinterpret_cast<const T2*>(smem);
+  double* H = smem + (MIXED ? 1 : 2) * d * kBins;  // a constant address where D is one
+  const JacGroups<T> cs = jacobian_groups<T, FAM>(it.fn, d, nullptr);
+  Integrand<T, FAM> F(it.fn);
+  const auto add = [&](double tmp) {
+    acc += tmp;
+    acc2 += tmp * tmp;
+  };
+  if (it.train)
+    span_trips<BS, MIXED>(tile.count, [&](uint32_t k) {
+      if constexpr (MIXED)
+        add(event_mixed_pairs<FAM, false>(F, lo0 + k, hi, draw, key, d, tab, cs, H, nullptr, wscale));
+      else
+        add(event_f64<FAM, true, true, 0>(F, lo0 + k, hi, draw, key, groups, d, tab, cs, H, nullptr, wscale));
+    });
+  else
+    span_trips<BS, MIXED>(tile.count, [&](uint32_t k) {
+      if constexpr (MIXED)
+        add(event_mixed<FAM, false>(F, lo0 + k, hi, draw, key, groups, d, tab, cs, nullptr, nullptr, wscale));
+      else
+        add(event_f64<FAM, false, false, 0>(F, lo0 + k, hi, draw, key, groups, d, tab, cs, nullptr, nullptr, wscale));
+    });
+}
+
+// One span with pair histograms (fused_event.hpp), BS threads. LDS = the map
+// table (mixed: float2; FP64: double2 per bin), then the pair tables.
+// PER_DIM: one event body per n_dim, chosen here.
+template <int FAM, int BS, bool MIXED, bool PER_DIM>
+__device__ __forceinline__ void batch_span_pairs(const mv_batch_item& it, const mv_batch_tile& tile, uint32_t draw,
+                                                 const double* __restrict__ grids, double* __restrict__ rows,
+                                                 double* smem) {
+  using T = typename std::conditional<MIXED, float, double>::type;
+  using T2 = typename std::conditional<MIXED, float2, double2>::type;
+  const int d = it.n_dim;
+  // 16-byte aligned: 50 d * 8 is a multiple of 400
+  double2* H = reinterpret_cast<double2*>(smem + (MIXED ? 1 : 2) * d * kBins);
+  __syncthreads();  // the previous span is done with the LDS
+  build_table<T, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, reinterpret_cast<T2*>(smem));
+  if (it.train)
+    for (int i = threadIdx.x; i < pair_cells(d) / 2; i += BS) H[i] = make_double2(0.0, 0.0);
+  __syncthreads();
   double acc = 0.0, acc2 = 0.0;
-  if constexpr (MIXED) {
-    float2* tab = reinterpret_cast<float2*>(smem);
-    build_table<float, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab);
-    if (it.train) {
-      const int half = pair_cells(d) / 2;
-      for (int i = threadIdx.x; i < half; i += BS) reinterpret_cast<double2*>(H)[i] = make_double2(0.0, 0.0);
-    }
-    const JacGroups<float> cs = jacobian_groups<float, FAM>(it.fn, d, nullptr);
-    __syncthreads();
-    Integrand<float, FAM> F(it.fn);
-    if (it.train) {
-      for (int k = threadIdx.x; k < tile.count; k += BS) {
-        const double tmp = event_mixed_pairs<FAM, false>(F, lo0 + (uint32_t)k, hi, draw, key, d, tab,
-                                                         cs, H, nullptr, wscale);
-        acc += tmp;
-        acc2 += tmp * tmp;
-      }
-    } else {
-      for (int k = threadIdx.x; k < tile.count; k += BS) {
-        const double tmp = event_mixed<FAM, false>(F, lo0 + (uint32_t)k, hi, draw, key, groups, d, tab,
-                                                   cs, nullptr, nullptr, wscale);
-        acc += tmp;
-        acc2 += tmp * tmp;
-      }
-    }
+#define MV_BTP(D) case D: batch_span_events<FAM, BS, MIXED, D>(it, tile, draw, smem, acc, acc2); break
+  if constexpr (!PER_DIM) {
+    batch_span_events<FAM, BS, MIXED, 0>(it, tile, draw, smem, acc, acc2);
   } else {
-    double2* tab = reinterpret_cast<double2*>(smem);
-    build_table<double, FAM>(it.fn, grids + it.grid_offset, d, nullptr, nullptr, tab);
-    const JacGroups<double> cs = jacobian_groups<double, FAM>(it.fn, d, nullptr);
-    if (it.train)
-      for (int i = threadIdx.x; i < pair_cells(d); i += BS) H[i] = 0.0;
-    __syncthreads();
-    Integrand<double, FAM> F(it.fn);
-    if (it.train) {
-      for (int k = threadIdx.x; k < tile.count; k += BS) {
-        const double tmp = event_f64<FAM, true, true, 0>(F, lo0 + (uint32_t)k, hi, draw, key, groups, d,
-                                                          tab, cs, H, nullptr, wscale);
-        acc += tmp;
-        acc2 += tmp * tmp;
-      }
-    } else {
-      for (int k = threadIdx.x; k < tile.count; k += BS) {
-        const double tmp = event_f64<FAM, false, false, 0>(F, lo0 + (uint32_t)k, hi, draw, key, groups, d,
-                                                            tab, cs, nullptr, nullptr, wscale);
-        acc += tmp;
-        acc2 += tmp * tmp;
-      }
+    switch (d) {
+      MV_BTP(1); MV_BTP(2); MV_BTP(3); MV_BTP(4); MV_BTP(5); MV_BTP(6); MV_BTP(7);
+      MV_BTP(8); MV_BTP(9); MV_BTP(10); MV_BTP(11); MV_BTP(12); MV_BTP(13);
+      default: batch_span_events<FAM, BS, MIXED, kPairMaxDim>(it, tile, draw, smem, acc, acc2); break;
     }
   }
-  finish_pairs<BS, true, MIXED>(acc, acc2, H, it.train ? d : 0, rows + it.row_offset);
+#undef MV_BTP
+  static_assert(kPairMaxDim == 14, "the switch above covers n_dim 1..14");
+  finish_pairs<BS, true, MIXED>(acc, acc2, reinterpret_cast<double*>(H), it.train ? d : 0, rows + it.row_offset);
+}
+
+// Cost of a training event for the split of the tiles (tiles.hpp), fitted to
+// the times of Gaussian events of one n_dim without the launch's fixed part
+// (17 us mixed, 22 us FP64): mixed, 5.12e7 events in 256 items, 79, 110, 99,
+// 154, 152, 187, 182, 228, 268 us at d = 2, 3, 4, 5, 6, 7, 8, 10, 12; FP64,
+// 1.28e7 events, 40, 50, 55, 79, 82, 91, 94, 122, 125, 138, 169 us at d = 2 ..
+// 10, 12, 14; within 6 %. The unpaired dimension of an odd n_dim has 50 cells
+// for all lanes.
+template <bool MIXED>
+__device__ __forceinline__ int batch_event_cost(int d) {
+  const int groups = (d + 3) >> 2, odd = d & 1;
+  return MIXED ? 23 * groups + 14 * d + 26 + 20 * odd : 56 * groups + 26 * d + 52 + 20 * odd;
 }
 
 template <int FAM, int BS, bool MIXED>
-__global__ __launch_bounds__(BS) void batch_fused_pairs(const mv_batch_item* __restrict__ items,
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4, 4))) void batch_fused_pairs(const mv_batch_item* __restrict__ items,
                                                         const mv_batch_tile* __restrict__ tiles,
-                                                        int n_tiles, int nbmax,
+                                                        int n_tiles,
                                                         const int32_t* __restrict__ draws,
                                                         const double* __restrict__ grids,
                                                         double* __restrict__ rows) {
   extern __shared__ double smem[];
-  for (int t = blockIdx.x; t < n_tiles; t += gridDim.x) {
-    const mv_batch_tile tile = tiles[t];
-    const mv_batch_item& it = items[tile.item];
-    const uint32_t draw = (uint32_t)draws[tile.item];
+  const auto work = [&](int i) {
+    const mv_batch_tile t = tiles[i];
+    return TileWork{t.item, t.count, t.first, batch_event_cost<MIXED>(items[t.item].n_dim),
+                    tile_begins(tiles, i)};
+  };
+  for_each_span<BS>(n_tiles, work, [&](int item, int64_t first, int count) {
+    const mv_batch_tile tile{item, count, first};
+    const mv_batch_item& it = items[item];
+    const uint32_t draw = (uint32_t)draws[item];
     if constexpr (FAM >= 0) {
-      // one event body per n_dim 1..kPairMaxDim, chosen per tile
-#define MV_BTP(D) case D: batch_tile_pairs<FAM, BS, MIXED, D>(it, tile, draw, grids, rows, smem, nbmax); break
-      switch (it.n_dim) {
-        MV_BTP(1); MV_BTP(2); MV_BTP(3); MV_BTP(4); MV_BTP(5); MV_BTP(6); MV_BTP(7);
-        MV_BTP(8); MV_BTP(9); MV_BTP(10); MV_BTP(11); MV_BTP(12); MV_BTP(13); MV_BTP(14);
-        default: batch_tile_pairs<FAM, BS, MIXED>(it, tile, draw, grids, rows, smem, nbmax); break;
-      }
-#undef MV_BTP
-      static_assert(kPairMaxDim == 14, "the switch above covers n_dim 1..14");
+      batch_span_pairs<FAM, BS, MIXED, true>(it, tile, draw, grids, rows, smem);
     } else {
       switch (it.fn.family) {
-        case MV_FN_CONSTANT: batch_tile_pairs<MV_FN_CONSTANT, BS, MIXED>(it, tile, draw, grids, rows, smem, nbmax); break;
-        case MV_FN_GAUSSIAN: batch_tile_pairs<MV_FN_GAUSSIAN, BS, MIXED>(it, tile, draw, grids, rows, smem, nbmax); break;
-        case MV_FN_PRODUCT: batch_tile_pairs<MV_FN_PRODUCT, BS, MIXED>(it, tile, draw, grids, rows, smem, nbmax); break;
-        case MV_FN_GAUSSMIX: batch_tile_pairs<MV_FN_GAUSSMIX, BS, MIXED>(it, tile, draw, grids, rows, smem, nbmax); break;
-        default: batch_tile_pairs<MV_FN_BWPOWER, BS, MIXED>(it, tile, draw, grids, rows, smem, nbmax); break;
+        case MV_FN_CONSTANT: batch_span_pairs<MV_FN_CONSTANT, BS, MIXED, false>(it, tile, draw, grids, rows, smem); break;
+        case MV_FN_GAUSSIAN: batch_span_pairs<MV_FN_GAUSSIAN, BS, MIXED, false>(it, tile, draw, grids, rows, smem); break;
+        case MV_FN_PRODUCT: batch_span_pairs<MV_FN_PRODUCT, BS, MIXED, false>(it, tile, draw, grids, rows, smem); break;
+        case MV_FN_GAUSSMIX: batch_span_pairs<MV_FN_GAUSSMIX, BS, MIXED, false>(it, tile, draw, grids, rows, smem); break;
+        default: batch_span_pairs<MV_FN_BWPOWER, BS, MIXED, false>(it, tile, draw, grids, rows, smem); break;
       }
     }
-  }
+  });
 }
 
 __global__ __launch_bounds__(64) void batch_finalize_kernel(const mv_batch_item* __restrict__ items,
@@ -304,25 +343,27 @@ size_t batch_pairs_lds(int max_dim, bool mixed) {
   return lds <= max_lds_per_block() ? lds : 0;
 }
 
-template <int F, bool MIXED>
-const void* batch_pairs_kernel() {
-  return reinterpret_cast<const void*>(batch_fused_pairs<F, kBatchPairBlock, MIXED>);
+using BatchPairsKernel = void (*)(const mv_batch_item*, const mv_batch_tile*, int, const int32_t*, const double*,
+                                  double*);
+
+template <bool MIXED>
+BatchPairsKernel batch_pairs_kernel(int family) {
+  switch (family) {
+    case MV_FN_CONSTANT: return batch_fused_pairs<MV_FN_CONSTANT, kBatchPairBlock, MIXED>;
+    case MV_FN_GAUSSIAN: return batch_fused_pairs<MV_FN_GAUSSIAN, kBatchPairBlock, MIXED>;
+    case MV_FN_PRODUCT: return batch_fused_pairs<MV_FN_PRODUCT, kBatchPairBlock, MIXED>;
+    case MV_FN_GAUSSMIX: return batch_fused_pairs<MV_FN_GAUSSMIX, kBatchPairBlock, MIXED>;
+    case MV_FN_BWPOWER: return batch_fused_pairs<MV_FN_BWPOWER, kBatchPairBlock, MIXED>;
+    default: return batch_fused_pairs<-1, kBatchPairBlock, MIXED>;
+  }
 }
 
 template <bool MIXED>
 int32_t pairs_blocks(int32_t family, int32_t max_dim) {
   const size_t lds = batch_pairs_lds(max_dim, MIXED);
   if (!lds) return 0;
-  const void* k = nullptr;
-  switch (family) {
-    case MV_FN_CONSTANT: k = batch_pairs_kernel<MV_FN_CONSTANT, MIXED>(); break;
-    case MV_FN_GAUSSIAN: k = batch_pairs_kernel<MV_FN_GAUSSIAN, MIXED>(); break;
-    case MV_FN_PRODUCT: k = batch_pairs_kernel<MV_FN_PRODUCT, MIXED>(); break;
-    case MV_FN_GAUSSMIX: k = batch_pairs_kernel<MV_FN_GAUSSMIX, MIXED>(); break;
-    case MV_FN_BWPOWER: k = batch_pairs_kernel<MV_FN_BWPOWER, MIXED>(); break;
-    default: k = batch_pairs_kernel<-1, MIXED>(); break;
-  }
-  return resident_blocks(k, lds, kBatchPairBlock);
+  return resident_blocks(reinterpret_cast<const void*>(batch_pairs_kernel<MIXED>(family)), lds,
+                         kBatchPairBlock);
 }
 
 template <bool MIXED>
@@ -335,20 +376,9 @@ int fused_pairs(const mv_batch_item* items, int32_t n_items, const mv_batch_tile
   const size_t lds = batch_pairs_lds(max_dim, MIXED);
   if (!lds) return fail(MV_ERR_UNSUPPORTED, "%s: max_dim must be 1..%d and fit the LDS", what, kPairMaxDim);
   if (blocks < 1) return fail(MV_ERR_ARG, "%s: blocks < 1", what);
-  const int nbmax = max_dim * kBins;
   hipStream_t s = as_stream(stream);
-#define MV_BP(F)                                                                                     \
-  hipLaunchKernelGGL((batch_fused_pairs<F, kBatchPairBlock, MIXED>), dim3(blocks), dim3(kBatchPairBlock), \
-                     lds, s, items, tiles, n_tiles, nbmax, draws, grids, rows)
-  switch (family) {
-    case MV_FN_CONSTANT: MV_BP(MV_FN_CONSTANT); break;
-    case MV_FN_GAUSSIAN: MV_BP(MV_FN_GAUSSIAN); break;
-    case MV_FN_PRODUCT: MV_BP(MV_FN_PRODUCT); break;
-    case MV_FN_GAUSSMIX: MV_BP(MV_FN_GAUSSMIX); break;
-    case MV_FN_BWPOWER: MV_BP(MV_FN_BWPOWER); break;
-    default: MV_BP(-1); break;
-  }
-#undef MV_BP
+  hipLaunchKernelGGL(batch_pairs_kernel<MIXED>(family), dim3(blocks), dim3(kBatchPairBlock), lds, s, items,
+                     tiles, n_tiles, draws, grids, rows);
   return check_launch(what);
 }
 }  // namespace

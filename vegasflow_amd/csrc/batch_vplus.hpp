@@ -3,14 +3,16 @@
 // persistent launch (vflowplus.py:37-80 + 187-220 per item). The iteration
 // end of the items is in vplus.hip (mv_batch_vplus_finalize).
 //
-// Workgroups stride over tiles of consecutive events of one item. Per tile:
-// the item's map table in LDS, histograms zeroed, then
-// the tile's 64-event trips split evenly over the waves, each wave walking
-// its run with the single-integral event body (vplus_run: hypercube lookup
-// over the item's offsets, draws, map, integrand, per-cube segmented sums
-// into the item's ress / ress2). The histogram goes into the item's row with
-// atomics. A tile past the item's events of this iteration (tiles cover an
-// upper bound of the adaptive event count) does nothing. Launches whose
+// Tiles of consecutive events of one item are split evenly over the
+// workgroups (tiles.hpp; eight mixtures of d = 4, two of 2e7 and six of 1e6
+// events requested: 276 us per launch with whole tiles dealt out in turn, 256
+// with the split, 240 with paced waves too). Per span: the item's map table in
+// LDS, histograms zeroed, then the span's 64-event trips split evenly over the
+// waves, each wave walking its run with the single-integral event body
+// (vplus_run: hypercube lookup over the item's offsets, draws, map, integrand,
+// per-cube segmented sums into the item's ress / ress2). The histogram goes
+// into the item's row with atomics. Tiles past the item's events of this iteration (tiles cover an
+// upper bound of the adaptive event count) have none. Launches whose
 // items share n_dim run a kernel compiled for it (the registers of one event
 // body); mixed dimensions choose the body per tile.
 #pragma once
@@ -24,6 +26,7 @@
 #include "device.hpp"
 #include "fused_event.hpp"
 #include "rows.hpp"
+#include "tiles.hpp"
 #include "vplus.hpp"
 #include "vplus_fused.hpp"
 
@@ -82,17 +85,23 @@ __global__ __launch_bounds__(BS) void batch_vplus_fused(const mv_batch_vplus_ite
   // or the pair tables)
   VplusEntry<MIXED>* tab = reinterpret_cast<VplusEntry<MIXED>*>(smem);
   double* hist = smem + 2 * nbmax;
-  for (int t = blockIdx.x; t < n_tiles; t += gridDim.x) {
-    const mv_batch_tile tile = tiles[t];
-    const mv_batch_vplus_item& it = items[tile.item];
+  // the events that the tiles have in this iteration
+  const auto work = [&](int i) {
+    const mv_batch_tile t = tiles[i];
+    const mv_batch_vplus_item& it = items[t.item];
+    const int64_t left = (int64_t)offsets[it.off_offset + it.n_cubes] - t.first;
+    const int groups = (it.n_dim + 3) >> 2;
+    return TileWork{t.item, (int)max((int64_t)0, min((int64_t)t.count, left)), t.first,
+                    MIXED ? 60 * groups + 21 * it.n_dim + 60 : 120 * groups + 33 * it.n_dim + 60,
+                    tile_begins(tiles, i)};
+  };
+  for_each_span<BS>(n_tiles, work, [&](int item, int64_t first, int count) {
+    const mv_batch_vplus_item& it = items[item];
     const StrataK st{it.n_strat, it.n_cubes, n_ev + it.cube_offset, offsets + it.off_offset};
-    const int64_t total = st.off[st.n_cubes];
-    const int64_t first = tile.first;
-    const int64_t end = min(first + (int64_t)tile.count, total);
-    if (first >= end) continue;  // workgroup-uniform: no barrier skipped by part of it
+    const int64_t end = first + count;
     const int d = it.n_dim;
     const int nb = d * kBins;
-    // this wave's run: the tile's trips split evenly over the waves
+    // this wave's run: the span's trips split evenly over the waves
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t trips = (end - first + 63) >> 6;
     const int64_t a = first + trip_of(wave, trips, W) * 64;
@@ -112,7 +121,7 @@ __global__ __launch_bounds__(BS) void batch_vplus_fused(const mv_batch_vplus_ite
     s.key.k1 = (uint32_t)(it.seed >> 32);
     s.xjac = 1.0 / (double)it.n_cubes;  // vflowplus.py:139
     s.xdeltajac = 1.0;
-    const uint32_t draw = (uint32_t)draws[tile.item];
+    const uint32_t draw = (uint32_t)draws[item];
     double* cr = ress + it.cube_offset;
     double* cr2 = ress2 + it.cube_offset;
     if constexpr (DSPEC > 0) {
@@ -135,7 +144,7 @@ __global__ __launch_bounds__(BS) void batch_vplus_fused(const mv_batch_vplus_ite
       else
         finish_row<true, false>(0.0, 0.0, hist, nb, rows + it.row_offset);
     }
-  }
+  });
 }
 
 using BatchVplusKernel = void (*)(const mv_batch_vplus_item*, const mv_batch_tile*, int, const int32_t*,
@@ -203,7 +212,7 @@ int launch_batch_vplus_precision(const mv_batch_vplus_item* items, const mv_batc
   // at most the workgroups resident at once (a persistent launch)
   const int res = resident_blocks(reinterpret_cast<const void*>(k), lds, bs);
   if (res < 1) return fail(MV_ERR_UNSUPPORTED, "mv_batch_vplus_fused: a workgroup does not fit (n_dim %d)", max_dim);
-  blocks = std::min(std::min(blocks, res), n_tiles);
+  blocks = std::min(blocks, res);
   hipLaunchKernelGGL(k, dim3(blocks), dim3(bs), lds, stream, items, tiles, n_tiles, draws, grids, n_ev, offsets,
                      ress, ress2, rows, nbmax);
   return check_launch("mv_batch_vplus_fused");
