@@ -104,7 +104,10 @@ typedef struct {
   int64_t event_offset;  /* global index of its first event */
   uint64_t seed;
   uint32_t draw_id;
-  uint32_t reserved2;
+  uint32_t iterations; /* 0 or 1: one; more: mv_vegas_fused without training and
+                        * mv_plain_fused run that many, drawing draw_id,
+                        * draw_id + 1, ...; iteration i adds into the group rows
+                        * rows + i * MV_ROWS * stride. No injected draws. */
   double xjac;           /* weight factor: 1/N (vegas, plain), 1/n_cubes (plus) */
   double xdeltajac;      /* prod(xmax - xmin), 1 without limits */
   const double* xmin;    /* nullable: integration limits (n_dim) */
@@ -140,7 +143,10 @@ typedef struct {
   int32_t train;         /* rows carry a histogram; refine the grid */
   int32_t refine;        /* apply the refinement to ``grid`` */
   int32_t raw;           /* write sum tmp^2 instead of sigma */
-  int32_t reserved;
+  int32_t iterations;    /* 0 or 1: one; more: those of a step with as many
+                          * (scalar, no training, not raw, with draw_dev): each
+                          * is recorded in its history slot, the last one's
+                          * results go to out, draw_dev[0] advances by them */
   double n_events;       /* N of the sigma formula */
   /* Iteration counter (nullable): draw_dev[0] is the draw id of the
    * iteration being finalized, draw_dev[1] a base. After the results,

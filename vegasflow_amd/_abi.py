@@ -64,7 +64,7 @@ class Step(ctypes.Structure):
         ("event_offset", _i64),
         ("seed", _u64),
         ("draw_id", _u32),
-        ("reserved2", _u32),
+        ("iterations", _u32),
         ("xjac", _f64),
         ("xdeltajac", _f64),
         ("xmin", _vp),
@@ -97,7 +97,7 @@ class Finalize(ctypes.Structure):
         ("train", _i32),
         ("refine", _i32),
         ("raw", _i32),
-        ("reserved", _i32),
+        ("iterations", _i32),
         ("n_events", _f64),
         ("draw_dev", _vp),
         ("history", _vp),

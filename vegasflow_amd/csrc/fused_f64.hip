@@ -20,7 +20,7 @@ namespace mv {
 template <int FAM, bool TRAIN, int D, bool INJ>
 __global__ __launch_bounds__(kBlock) void vegas_fused_f64(StepK s, mv_integrand fn,
                                                           const double* __restrict__ grid, RowsK R) {
-  const uint32_t draw = draw_of(s);
+  const uint32_t draw = iteration_draw(s);
   constexpr int nb = D * kBins;
   __shared__ __align__(16) double smem[(2 + (TRAIN ? kWaves : 0)) * nb];
   double2* tab = reinterpret_cast<double2*>(smem);
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kBlock) void vegas_fused_f64(StepK s, mv_integrand 
       acc2 += tmp * tmp;
     });
   }
-  finish_block<TRAIN>(acc, acc2, hist, nb, R);
+  finish_block<TRAIN>(acc, acc2, hist, nb, iteration_rows(R));
 }
 
 namespace {
@@ -75,7 +75,7 @@ int launch_fam(const StepK& k, const mv_integrand& fn, const double* grid, const
     return fail(MV_ERR_UNSUPPORTED, "fused FP64 kernel: n_dim %d outside 1..%d", k.n_dim,
                 MV_FUSED_MAX_DIM);
   const Kernel kern = (k.inject ? table_inj : table)[k.n_dim - 1];
-  return launch_producer(kern, k.n_events, 0, st, k, fn, grid, R);
+  return launch_iterations(kern, k, st, fn, grid, R);
 }
 
 }  // namespace

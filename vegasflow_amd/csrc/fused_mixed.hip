@@ -22,7 +22,7 @@ namespace mv {
 template <int FAM, bool TRAIN, int D, bool INJ>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(TRAIN ? 2 : 8))) void vegas_fused_mixed(
     StepK s, mv_integrand fn, const double* __restrict__ grid, RowsK R) {
-  const uint32_t draw = draw_of(s);
+  const uint32_t draw = iteration_draw(s);
   constexpr int nb = D * kBins;
   __shared__ __align__(16) double smem[(1 + (TRAIN ? kWaves : 0)) * nb];  // static: constant addresses
   float2* tab = reinterpret_cast<float2*>(smem);  // nb float2
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(TRAIN ? 
       acc2 += tmp * tmp;
     });
   }
-  finish_block<TRAIN>(acc, acc2, hist, nb, R);
+  finish_block<TRAIN>(acc, acc2, hist, nb, iteration_rows(R));
 }
 
 namespace {
@@ -77,7 +77,7 @@ int launch_fam(const StepK& k, const mv_integrand& fn, const double* grid, const
     return fail(MV_ERR_UNSUPPORTED, "fused mixed kernel: n_dim %d outside 1..%d", k.n_dim,
                 MV_FUSED_MAX_DIM);
   const Kernel kern = (k.inject ? table_inj : table)[k.n_dim - 1];
-  return launch_producer(kern, k.n_events, 0, st, k, fn, grid, R);
+  return launch_iterations(kern, k, st, fn, grid, R);
 }
 
 }  // namespace

@@ -118,7 +118,7 @@ __device__ __forceinline__ void plain_events(const StepK& s, uint32_t draw, Inte
 
 template <int FAM, bool MIXED, int D, bool INJ>
 __global__ __launch_bounds__(kBlock) void plain_fused(StepK s, mv_integrand fn, RowsK R) {
-  const uint32_t draw = draw_of(s);
+  const uint32_t draw = iteration_draw(s);
   using T = typename std::conditional<MIXED, float, double>::type;
   Integrand<T, FAM> F(fn);
   const bool limits = s.xmin != nullptr;
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(kBlock) void plain_fused(StepK s, mv_integrand fn, 
   } else {
     plain_events<FAM, MIXED, D, INJ, false>(s, draw, F, wt, acc, acc2);
   }
-  finish_block<false>(acc, acc2, nullptr, 0, R);
+  finish_block<false>(acc, acc2, nullptr, 0, iteration_rows(R));
 }
 
 namespace {
@@ -156,7 +156,7 @@ int launch_fam(const StepK& k, const mv_integrand& fn, const RowsK& R, hipStream
   const Kernel kern = k.n_dim >= 1 && k.n_dim <= MV_FUSED_MAX_DIM
                           ? (inj ? table_inj : table)[k.n_dim - 1]
                           : (inj ? &plain_fused<FAM, MIXED, 0, true> : &plain_fused<FAM, MIXED, 0, false>);
-  return launch_producer(kern, k.n_events, 0, st, k, fn, R);
+  return launch_iterations(kern, k, st, fn, R);
 }
 
 }  // namespace

@@ -350,6 +350,8 @@ __global__ __launch_bounds__(kBlock) void vegas_digest(StepK s, const FT* __rest
 // ---------------------------------------------------------------------------
 // finalize: block 0 sums and sigma, block 1 + j dimension j (refine.hpp)
 // ---------------------------------------------------------------------------
+constexpr int kIterationsBlock = 1024;
+
 __global__ __launch_bounds__(kBlock) void finalize_kernel(FzK z, double* __restrict__ P,
                                                           int64_t stride, int nrows,
                                                           double* __restrict__ grid,
@@ -359,6 +361,49 @@ __global__ __launch_bounds__(kBlock) void finalize_kernel(FzK z, double* __restr
     finalize_sums_block(z, P, stride, nrows, out);
   else
     hist_refine_block(z, P, stride, nrows, (int)blockIdx.x - 1, grid, hist_out);
+}
+
+// Ends of z.iterations iterations without a histogram (n_out = 1): a wave per
+// iteration, whose two columns of MV_ROWS rows it reads at once and sums in
+// each half wave, as finalize_sums_block does.
+__global__ __launch_bounds__(kIterationsBlock) void finalize_iterations(FzK z, int iterations,
+                                                                        double* __restrict__ P, int64_t stride,
+                                                                        int nrows, double* __restrict__ out) {
+  static_assert(MV_ROWS == 32, "a half wave holds a column");
+  const int lane = threadIdx.x & 63, row = lane & 31;
+  const uint32_t slot = z.counter.draw[0] - z.counter.draw[1];
+  for (int i = threadIdx.x >> 6; i < iterations; i += kIterationsBlock / 64) {
+    double v = 0.0;
+    if (row < nrows) {
+      double* p = P + ((int64_t)i * MV_ROWS + row) * stride + (lane >> 5);
+      v = *p;
+      *p = 0.0;
+    }
+    v += dpp_f64<0xB1, 0xF, true>(v);   // quad_perm [1, 0, 3, 2]
+    v += dpp_f64<0x4E, 0xF, true>(v);   // quad_perm [2, 3, 0, 1]
+    v += dpp_f64<0x124, 0xF, true>(v);  // row_ror 4
+    v += dpp_f64<0x128, 0xF, true>(v);  // row_ror 8
+    v += dpp_f64<0x142, 0xA>(v);        // row_bcast 15 into rows 1 and 3
+    const double res = bcast_lane(v, 31), res2 = bcast_lane(v, 63);
+    if (lane == 0) {
+      const double N = z.n_events;
+      const double sig = sqrt_clamped((N * res2 - res * res) / (N - 1.0));  // vflow.py:437-438
+      flag_nonfinite(z.status, res, res2);
+      const uint32_t k = slot + (uint32_t)i;
+      if (z.counter.history && k < (uint32_t)z.counter.len) {
+        double* h = z.counter.history + 3 * (int64_t)k;
+        h[0] = res;
+        h[1] = sig;
+        h[2] = N;
+      }
+      if (i == iterations - 1) {
+        out[0] = res;
+        out[1] = sig;
+      }
+    }
+  }
+  __syncthreads();  // every wave has read the counter
+  if (threadIdx.x == 0) z.counter.draw[0] += (uint32_t)iterations;
 }
 
 __global__ __launch_bounds__(64) void refine_kernel(const double* __restrict__ hist, int64_t hstride,
@@ -443,6 +488,15 @@ extern "C" int32_t mv_producer_rows(int64_t n_events) {
 
 namespace {
 
+// Several iterations in one launch: no training, no injected draws, and at most
+// as many as a grid has in its second dimension.
+int validate_iterations(const mv_step* s, const char* what, bool train) {
+  if (s->iterations <= 1) return MV_OK;
+  if (train || s->inject) return fail(MV_ERR_ARG, "%s: several iterations need a step without training and inject", what);
+  if (s->iterations > 65535) return fail(MV_ERR_UNSUPPORTED, "%s: more than 65535 iterations", what);
+  return MV_OK;
+}
+
 // Whether a training step runs through pair tables: their LDS (static in the
 // kernels: the map table, then the cells) must be what a workgroup may have.
 bool pairs_apply(int d, bool mixed) {
@@ -481,6 +535,7 @@ extern "C" int mv_vegas_fused(const mv_step* step, const mv_integrand* fn, const
   if (rc) return rc;
   if ((rc = validate_fn(fn, "mv_vegas_fused"))) return rc;
   if (!grid) return fail(MV_ERR_ARG, "mv_vegas_fused: grid is required");
+  if ((rc = validate_iterations(step, "mv_vegas_fused", step->train != 0))) return rc;
   RowsK R;
   if ((rc = make_rows(parts, mv_partial_stride(step->n_dim, 1, step->train),
                       "mv_vegas_fused", &R)))
@@ -506,6 +561,7 @@ extern "C" int mv_plain_fused(const mv_step* step, const mv_integrand* fn, const
   int rc = validate_step(step, "mv_plain_fused", 0);
   if (rc) return rc;
   if ((rc = validate_fn(fn, "mv_plain_fused"))) return rc;
+  if ((rc = validate_iterations(step, "mv_plain_fused", false))) return rc;
   if ((fn->family == MV_FN_GAUSSIAN || fn->family == MV_FN_GAUSSMIX) &&
       step->n_dim > MV_FUSED_MAX_DIM)
     return fail(MV_ERR_UNSUPPORTED, "mv_plain_fused: n_dim %d exceeds %d for this family",
@@ -648,6 +704,13 @@ extern "C" int mv_vegas_finalize(const mv_finalize* fz, double* rows, int64_t ro
   if (fz->history && fz->history_len < 0) return fail(MV_ERR_ARG, "mv_vegas_finalize: history_len < 0");
   FzK z{fz->n_dim, fz->n_out, fz->train, fz->refine, fz->raw, fz->n_events,
         CounterK{fz->draw_dev, fz->history, fz->history_len}, fz->status};
+  if (fz->iterations > 1) {
+    if (fz->train || fz->refine || fz->raw || fz->n_out != 1 || !fz->draw_dev)
+      return fail(MV_ERR_ARG, "mv_vegas_finalize: several iterations need a counter, one output and no training");
+    hipLaunchKernelGGL(finalize_iterations, dim3(1), dim3(kIterationsBlock), 0, as_stream(stream), z, fz->iterations,
+                       rows, row_stride, n_rows, out);
+    return check_launch("mv_vegas_finalize");
+  }
   const int blocks = 1 + (fz->train ? fz->n_dim : 0);  // histogram columns are always consumed
   hipLaunchKernelGGL(finalize_kernel, dim3(blocks), dim3(kBlock), 0, as_stream(stream), z, rows,
                      row_stride, n_rows, grid, out, hist_out);
@@ -741,6 +804,7 @@ extern "C" int mv_vegas_iteration_static(const mv_step* step, const mv_integrand
   if (rc) return rc;
   if ((rc = validate_fn(fn, "mv_vegas_iteration_static"))) return rc;
   if (step->n_events < 1) return fail(MV_ERR_ARG, "mv_vegas_iteration_static: n_events must be >= 1");
+  if (step->iterations > 1) return fail(MV_ERR_ARG, "mv_vegas_iteration_static: one iteration per call");
   if (!grid || !out) return fail(MV_ERR_ARG, "mv_vegas_iteration_static: grid and out are required");
   if ((refine || hist_out) && !step->train)
     return fail(MV_ERR_ARG, "mv_vegas_iteration_static: refine and hist_out need a training step");

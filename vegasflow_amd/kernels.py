@@ -128,10 +128,11 @@ class Workspace:
     when allocated; producers add into them and the finalize calls consume
     and re-zero them."""
 
-    def __init__(self, device, stride):
+    def __init__(self, device, stride, iterations=1):
         self.device = device
         self.stride = int(stride)
-        self.rows = torch.zeros(_abi.ROWS * self.stride, dtype=torch.float64, device=device)
+        self.iterations = int(iterations)  # that one producer call may run
+        self.rows = torch.zeros(self.iterations * _abi.ROWS * self.stride, dtype=torch.float64, device=device)
         self._struct = _abi.Partials(self.rows.data_ptr(), self.stride)
 
     def partials(self):
@@ -164,7 +165,7 @@ def producer_rows(n_events):
 
 def make_step(n_dim, n_events, *, precision="f64", train=True, event_offset=0,
               seed=0, draw_id=0, xjac=1.0, xmin=None, xdelta=None, xdeltajac=1.0, inject=None,
-              draw_dev=None):
+              draw_dev=None, iterations=1):
     _need_device(xmin, "xmin", torch.float64)
     _need_device(draw_dev, "draw_dev", torch.int32)
     _need_device(xdelta, "xdelta", torch.float64)
@@ -183,6 +184,7 @@ def make_step(n_dim, n_events, *, precision="f64", train=True, event_offset=0,
     s.event_offset = int(event_offset)
     s.seed = int(seed) & 0xFFFFFFFFFFFFFFFF
     s.draw_id = int(draw_id) & 0xFFFFFFFF
+    s.iterations = int(iterations)
     s.xjac = float(xjac)
     s.xdeltajac = float(xdeltajac)
     s.xmin = None if xmin is None else xmin.data_ptr()
@@ -282,11 +284,17 @@ class IterationCounter:
 # ---------------------------------------------------------------------------
 # VegasFlow / PlainFlow
 # ---------------------------------------------------------------------------
+def _rows_for(step, ws):
+    if step.iterations > ws.iterations:
+        raise ValueError(f"the workspace has rows for {ws.iterations} iterations, the step {step.iterations}")
+    return ws.partials()
+
+
 def vegas_fused(step, fn_struct, grid, ws):
     """mv_vegas_fused; returns the number of group rows of ``ws`` touched."""
     _need_device(grid, "grid", torch.float64)
     return _call("mv_vegas_fused", ctypes.byref(step), ctypes.byref(fn_struct), _ptr(grid),
-                     ws.partials(), _stream())
+                     _rows_for(step, ws), _stream())
 
 
 def vegas_iteration_static(step, fn_struct, grid, refine, out, hist_out=None, status=None):
@@ -306,7 +314,7 @@ def vegas_iteration_static(step, fn_struct, grid, refine, out, hist_out=None, st
 
 
 def plain_fused(step, fn_struct, ws):
-    return _call("mv_plain_fused", ctypes.byref(step), ctypes.byref(fn_struct), ws.partials(),
+    return _call("mv_plain_fused", ctypes.byref(step), ctypes.byref(fn_struct), _rows_for(step, ws),
                      _stream())
 
 
@@ -350,11 +358,14 @@ def vegas_digest(step, f, w, idx, ws, main_dim=0):
 
 
 def vegas_finalize(n_dim, n_out, train, refine, n_events, ws, n_rows, grid=None, hist_out=None,
-                   raw=False, counter=None, status=None):
+                   raw=False, counter=None, status=None, iterations=1):
     """Reduce group rows; returns a (2 * n_out,) float64 tensor [res, sigma]
     (or [res, sum tmp^2] with raw). ``counter``: an IterationCounter the
     kernel records the result in and advances. ``status``: an int32 device
-    word the kernel ORs MV_STATUS_NONFINITE into for non-finite sums."""
+    word the kernel ORs MV_STATUS_NONFINITE into for non-finite sums.
+    ``iterations``: of the step (needs a counter)."""
+    if iterations > ws.iterations:
+        raise ValueError(f"the workspace has rows for {ws.iterations} iterations, not {iterations}")
     out = torch.empty(2 * n_out, dtype=torch.float64, device=ws.device)
     _need_device(grid, "grid", torch.float64)
     _need_device(hist_out, "hist_out", torch.float64)
@@ -365,6 +376,7 @@ def vegas_finalize(n_dim, n_out, train, refine, n_events, ws, n_rows, grid=None,
     fz.refine = int(bool(refine))
     fz.raw = int(bool(raw))
     fz.n_events = float(n_events)
+    fz.iterations = int(iterations)
     if counter is not None:
         fz.draw_dev = counter.draw.data_ptr()
         fz.history = counter.history.data_ptr()

@@ -63,6 +63,17 @@ class PlainFlow(MonteCarloFlow):
         kernels.vegas_finalize(self.n_dim, 1, False, False, n, ws, ng, counter=counter,
                                status=counter.status)
 
+    def _independent_iterations(self):
+        return True
+
+    def _graph_group(self, counter, n_iter):
+        n = self.n_events
+        ws = self._group_workspace()
+        step = self._step(n, train=False, offset=0, draw_dev=counter.draw, iterations=n_iter)
+        ng = kernels.plain_fused(step, self._fused, ws)
+        kernels.vegas_finalize(self.n_dim, 1, False, False, n, ws, ng, counter=counter, status=counter.status,
+                               iterations=n_iter)
+
     def _fused_iteration(self, inject=None):
         self._next_draw()
         n = self.n_events

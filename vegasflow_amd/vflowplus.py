@@ -248,6 +248,9 @@ class VegasFlowPlus(VegasFlow):
                 self._offsets.data_ptr(), self._ress.data_ptr(), self._ress2.data_ptr(), ws.rows.data_ptr(),
                 None if xmin is None else xmin.data_ptr(), None if xdelta is None else xdelta.data_ptr())
 
+    def _independent_iterations(self):
+        return False  # the allocation of events follows the last iteration
+
     def _graph_iteration(self, counter):
         ws = self._workspace_for(kernels.partial_stride(self.n_dim, 1, self.train))
         step = self._step(self._events_bound(), train=self.train, offset=0, xjac=self._modified_jac,
