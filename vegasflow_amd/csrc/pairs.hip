@@ -16,6 +16,16 @@
 
 namespace mv {
 
+// Whether one workgroup fills a CU, by its LDS (from d = 7) or its registers
+// (the mixture from d = 4): its waves are then paced (paced_trips). Mixture, 1e7
+// events, without and with: 32.5 and 30.4 us at d = 4, 45.4 and 42.9 at 5, 48.0
+// and 44.9 at 6; Gaussian, two workgroups per CU: 24.0 and 25.4 us at d = 4,
+// 34.8 and 36.5 at 6.
+template <int FAM, int D>
+constexpr bool pairs_paced() {
+  return D > 6 || (FAM == MV_FN_GAUSSMIX && D >= 4);
+}
+
 template <int FAM, int D>
 __global__ __launch_bounds__(kPairBlock) void vegas_fused_pairs(StepK s, mv_integrand fn,
                                                                 const double* __restrict__ grid,
@@ -47,7 +57,7 @@ __global__ __launch_bounds__(kPairBlock) void vegas_fused_pairs(StepK s, mv_inte
       acc2 += tmp * tmp;
     }
   } else {
-    event_trips<kPairBlock, (D > 6)>(s, [&](uint32_t c) {
+    event_trips<kPairBlock, pairs_paced<FAM, D>()>(s, [&](uint32_t c) {
       const double tmp = event_mixed_pairs<FAM, false>(F, c, s.ev_hi, draw, s.key, D, tab, cs, H, nullptr,
                                                        wscale);
       acc += tmp;
