@@ -110,18 +110,6 @@ constexpr int kPairBlock = 1024;  // threads of a pair-histogram workgroup
 
 __host__ __device__ constexpr int pair_cells(int d) { return ((d + 1) >> 1) * kPairBins; }
 
-// cell (b_2p, b_2p+1) of pair p gets tmp2; b_2p+1 = 0 (its byte of pk is
-// never set) for the unpaired last dimension of an odd d
-__device__ __forceinline__ void pair_adds(double* H, const uint32_t (&pk)[4], int d, double tmp2) {
-#pragma unroll
-  for (int p = 0; p < kPairMaxDim / 2; ++p) {
-    if (2 * p < d) {
-      const uint32_t w = pk[p >> 1] >> (16 * (p & 1));
-      lds_add(&H[p * kPairBins + (w & 0xffu) * kBins + ((w >> 8) & 0xffu)], tmp2);
-    }
-  }
-}
-
 // Bin b of dimension j = m / 50 (b = m % 50) from the pair histograms is the
 // sum of row b of pair j / 2 for an even j, of column b for an odd j. This is
 // half h of that sum (h = 0: cells 0..24, h = 1: cells 25..49) in order; the
@@ -136,8 +124,9 @@ __device__ __forceinline__ double pair_marginal_half(const double* H, int m, int
   return a;
 }
 
-// The same from the byte offset of the event's cell within each pair table
-// (one multiply-add per pair of dimensions, no packed bins to take apart).
+// tmp2 into the event's cell of every pair table, from the cell's byte offset
+// within it (one multiply-add per pair of dimensions; the second bin of the
+// unpaired last dimension of an odd d is 0).
 template <int N>
 __device__ __forceinline__ void pair_cell_adds(double* H, const uint32_t (&cell)[N], int d, double tmp2) {
   char* Hb = reinterpret_cast<char*>(H);

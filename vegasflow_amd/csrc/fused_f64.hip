@@ -58,9 +58,18 @@ namespace {
 
 using Kernel = void (*)(StepK, mv_integrand, const double*, RowsK);
 
+// Training with kPairMinDim .. kPairMaxDim dimensions is the pair kernel's.
+template <int FAM, bool TRAIN, int D, bool INJ>
+constexpr Kernel kernel_at() {
+  if constexpr (TRAIN && D >= kPairMinDim && D <= kPairMaxDim)
+    return nullptr;
+  else
+    return &vegas_fused_f64<FAM, TRAIN, D, INJ>;
+}
+
 template <int FAM, bool TRAIN, bool INJ, int... Ds>
 constexpr std::array<Kernel, sizeof...(Ds)> kernels_of(std::integer_sequence<int, Ds...>) {
-  return {&vegas_fused_f64<FAM, TRAIN, Ds + 1, INJ>...};
+  return {kernel_at<FAM, TRAIN, Ds + 1, INJ>()...};
 }
 
 template <int FAM, bool TRAIN>
@@ -75,6 +84,7 @@ int launch_fam(const StepK& k, const mv_integrand& fn, const double* grid, const
     return fail(MV_ERR_UNSUPPORTED, "fused FP64 kernel: n_dim %d outside 1..%d", k.n_dim,
                 MV_FUSED_MAX_DIM);
   const Kernel kern = (k.inject ? table_inj : table)[k.n_dim - 1];
+  if (!kern) return fail(MV_ERR_UNSUPPORTED, "training n_dim %d needs the pair kernel's LDS", k.n_dim);
   return launch_iterations(kern, k, st, fn, grid, R);
 }
 
