@@ -240,13 +240,15 @@ __device__ __forceinline__ void event_trips(const StepK& s, Body&& body) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t w0 = ((int64_t)wave * gridDim.x + blockIdx.x) * 64;  // the wave's first event
   const int64_t i0 = w0 + (threadIdx.x & 63);
-  const int64_t full = s.n_events - 64 - w0 >= 0 ? (s.n_events - 64 - w0) / step + 1 : 0;
+  // at most 2^32 events in steps of 64 or more: the count is an int, which the
+  // scalar unit compares (64 bits take two VALU instructions per trip)
+  const int full = s.n_events - 64 - w0 >= 0 ? (int)((s.n_events - 64 - w0) / step) + 1 : 0;
   uint32_t c = s.ev_lo + (uint32_t)i0;
-  paced_trips<PACED, int64_t>(0, full, 1, [&](int64_t) {
+  paced_trips<PACED>(0, full, 1, [&](int) {
     body(c);
     c += (uint32_t)step;
   });
-  if (i0 + full * step < s.n_events) body(c);
+  if (i0 + (int64_t)full * step < s.n_events) body(c);
 }
 
 // Start of share g of ``trips`` split evenly over ``n`` (g = 0 .. n, n > 0): a
