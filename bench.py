@@ -34,7 +34,7 @@ PEAK = {"mixed": 157.3, "f64": 78.6}  # TFLOP/s, MI355X datasheet (FP32 / FP64 v
 # FETCH_SIZE and WRITE_SIZE passes of rocprofv3 scaled by a 1 GiB copy
 # (profiles/vegas_fused_gauss_d8_1e7_pmc.md): 0 bytes per event; the grid
 # reads and the FP64 atomic adds of the partial rows
-TRAFFIC = {"mixed": 0.9748e6, "f64": 0.9830e6}
+TRAFFIC = {"mixed": 1.0486e6, "f64": 1.0445e6}
 TRAFFIC_SOURCE = "profiles/vegas_fused_gauss_d8_1e7_pmc.md"
 # VALU wave instructions per launch (SQ_INSTS_VALU, same profile) and the
 # VALU-busy cycles per 64 events: the instruction classes of the counters
@@ -42,8 +42,8 @@ TRAFFIC_SOURCE = "profiles/vegas_fused_gauss_d8_1e7_pmc.md"
 # `bench.py --only issue` measures on gfx950 (2 cycles per wave64 FP32 add,
 # multiply or FMA, 8 per v_exp_f32, 4 for every other kind), set against
 # 4 SIMDs per CU at the 2.4 GHz engine clock (MI355X datasheet)
-VALU_INSTS = {"mixed": 2.351e7, "f64": 5.107e7}
-VALU_BUSY_CYCLES = {"mixed": 549.9, "f64": 1307.3}
+VALU_INSTS = {"mixed": 2.375e7, "f64": 4.159e7}
+VALU_BUSY_CYCLES = {"mixed": 556.0, "f64": 1064.6}
 VALU_SOURCE = "profiles/vegas_fused_gauss_d8_1e7_valu_mix.md"
 CLOCK_HZ = 2.4e9
 # host cores allotted to one GPU of the node (CPU worker pools are sized to it)

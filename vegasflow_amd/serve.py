@@ -125,9 +125,11 @@ class Server:
         self.precision = precision_of(DTYPE if dtype is None else dtype)
         # training goes through the pair-histogram batch kernel
         # (mv_batch_fused_pairs / _f64) wherever it takes the family's max
-        # n_dim: by default in mixed precision only (on the request mix of
-        # the serving benchmark the FP64 pair kernel raised the median
-        # latency, 4.4 -> 5.2 ms, for 3 % off the 99th percentile)
+        # n_dim: by default in mixed precision only (set when the FP64 pair
+        # kernel dealt out whole tiles and raised the median latency; since
+        # it splits the tile list, pair_histograms=True is the faster choice
+        # in FP64 too: bursts of 6, 10 and 16 requests 1.99 -> 1.71, 7.8 ->
+        # 7.1 and 12.6 -> 11.6 ms. The default is what callers rely on.)
         self.pairs = self.precision == "mixed" if pair_histograms is None else bool(pair_histograms)
         self.pair_events_per_tile = int(pair_events_per_tile)
         self.capacity = int(memory_budget // slot_bytes())
