@@ -72,13 +72,15 @@ __device__ __forceinline__ double draw_f64(uint32_t hi, uint32_t lo) {
 
 // The position xn = 50 (1 - u) of the FP64 draw hi:lo in the unit interval of
 // 50 bins (vflow.py:117), for the fused kernels: 2 - m = 1 - r is exact, so
-// xn = fma(50 span, 1 - r, 50 (1 - TECH_CUT - span)) has one rounding where u,
+// xn = fma(50 span, 1 - r, 50 (1 - span - TECH_CUT)) has one rounding where u,
 // 1 - u and the product with 50 have four: two FP64 operations for five, and
-// nearer to the real number (against 80-bit arithmetic rms 2.7e-15 and at most
-// 5.8e-15, the four roundings 2.9e-15 and 8.0e-15; the bins of the two forms
+// nearer to the real number (against exact arithmetic rms 1.4e-15 and at most
+// 4.0e-15, the four roundings 2.9e-15 and 8.0e-15; the bins of the two forms
 // differ only where xn is within that of an edge). Always inside (0, 50).
 __device__ __forceinline__ double position_f64(uint32_t hi, uint32_t lo) {
-  constexpr double kEnd = kFBins * ((1.0 - kTechCut) - kSpan);  // xn of r = 1: 50 TECH_CUT
+  // xn of r = 1, about 50 TECH_CUT. 1 - span is exact, so this order leaves no
+  // error that counts; (1 - TECH_CUT) - span would shift every position by 2.5e-15
+  constexpr double kEnd = kFBins * ((1.0 - kSpan) - kTechCut);
   return fma(2.0 - draw_mantissa(hi, lo), kFBins * kSpan, kEnd);
 }
 
