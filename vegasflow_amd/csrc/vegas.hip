@@ -70,7 +70,8 @@ size_t max_lds_per_block() {
 }
 
 // ---------------------------------------------------------------------------
-// unfused path: sample (any n_dim)
+// unfused path: sample (any n_dim; Philox draws up to MV_FUSED_MAX_DIM
+// dimensions run the kernels of sample.hip)
 // With STAGED, each block writes its 256 events' rows of x (and bins) to LDS
 // first and then stores the block's contiguous part of the row-major (n, d)
 // outputs with consecutive threads on consecutive elements (full cache lines

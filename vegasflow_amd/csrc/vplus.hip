@@ -5,7 +5,9 @@
 // offsets[c] .. offsets[c+1]-1 (offsets = exclusive prefix sum of n_ev,
 // vflowplus.py:67). A wave handles 64 consecutive events, so the cube ids in
 // a wave are sorted; per-cube sums are a segmented wave scan followed by one
-// FP64 global atomic per (wave, cube) segment.
+// FP64 global atomic per (wave, cube) segment. The sampler here takes injected
+// draws and n_dim > MV_FUSED_MAX_DIM, the digest frozen grids and n_dim outside
+// 2..14; the others are in sample.hip and digest.hip.
 #include <algorithm>
 #include <type_traits>
 
